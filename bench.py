@@ -548,14 +548,17 @@ def main():
         }
 
     def roof(st, mixed):
-        name = "gm_lat_ana_s_mixed" if mixed else "gm_lat_ana_s"
+        name = "gm_lat_ana_s_mixed" if mixed else "gm_lat2_ana"
         dom_ms = st.get(name, {}).get("mean_ms", float("nan"))
-        achieved = f2 / (dom_ms * 1e-3)
-        # 2 (2 + 4) FLOP per (l, m, ring): 4 of the recurrence (FP64), 8 of the contraction
-        # (FP64, or FP32 in the mixed kernel); the peak is the time-weighted one of that mix
+        # mixed: 2 (2 + 4) FLOP per (l, m, ring), 4 of the recurrence (FP64), 8 of the contraction
+        # (FP32), against the time-weighted peak of that mix.  FP64 (spin 2 on the spin-0 rows):
+        # 2 (2 + 4) per (l, m, ring pair)
+        flop = f2 if mixed else 2 * (2 + 4) * (lmax + 1) * (lmax + 2) / 2 * 2 * nside
+        achieved = flop / (dom_ms * 1e-3)
         peak = PEAK_FP64 if not mixed else 12.0 / (4.0 / PEAK_FP64 + 8.0 / PEAK_FP32)
         return {
-            "kernel": f"k_ana_s{'<mixed>' if mixed else ''} (spin-2 Legendre analysis, {name})",
+            "kernel": (f"k_ana_s<mixed> (spin-2 Legendre analysis, {name})" if mixed else
+                       f"k_ana_pairs (spin-2 analysis on the spin-0 rows of ring pairs, {name})"),
             "bound": "valu",
             "pipe": ("FP64 VALU (MI355X FP64 vector and matrix peaks are both 78.6 TFLOP/s)" if not mixed else
                      "FP64 VALU recurrence (78.6 TFLOP/s) + FP32 VALU contraction (157.3 TFLOP/s): op-mix peak"),
@@ -563,8 +566,8 @@ def main():
             "peak": peak / 1e12,
             "unit": "TFLOP/s",
             "frac": achieved / peak,
-            "traffic": _measured_traffic(nside, "k_ana_s_mixed" if mixed else "k_ana_s"),
-            "flop_per_launch": f2,
+            "traffic": _measured_traffic(nside, "k_ana_s_mixed" if mixed else "k_ana_pairs"),
+            "flop_per_launch": flop,
             "mean_launch_ms": dom_ms,
         }
 

@@ -70,37 +70,16 @@ class BatPlan:
     res: tuple             # (jsplit, mpol, nb32, nb64, tsize64) of the FP16 hi/lo analysis
 
 
-def _nactive_pairs(nside, lmax, polar_skip):
-    """Ring pairs (equator first) that order m visits: the larger of ducc0's spin-0 and
-    spin-2 polar-skip bounds (``sht._nactive``), evaluated on the folded rings."""
-    z, sin = sht._ring_slots(nside, 0)
-    n = len(z)
-    L = lmax + 1
-    if not polar_skip:
-        return np.full(L, n, dtype=np.int32)
-    ofs = max(100.0, 0.01 * lmax)
-    b = lmax * sin + ofs
-    mlim0 = b
-    mlim2 = 2.0 * np.abs(z) + np.sqrt(np.maximum(b * b - 4.0 * sin * sin, 0.0))
-    best = np.maximum.accumulate(np.maximum(mlim0, mlim2)[::-1])[::-1]
-    return np.searchsorted(-best, -np.arange(L), side="right").astype(np.int32)
-
-
-def _split_at(nside, sin2):
-    _, sin = sht._ring_slots(nside, 0)
-    return int(np.count_nonzero(sin * sin >= sin2))
-
-
 def polar_split(nside):
     """Number of ring pairs (from the equator) with sin^2(theta) >= POLAR_SIN2."""
-    return _split_at(nside, POLAR_SIN2)
+    return sht._split_at(nside, POLAR_SIN2)
 
 
 def residual_split(nside):
     """First ring pair of the FP16 hi/lo analysis contracted in FP64 (RES_SIN2_RANGE)."""
-    lo, hi = _split_at(nside, RES_SIN2_RANGE[0]), _split_at(nside, RES_SIN2_RANGE[1])
+    lo, hi = sht._split_at(nside, RES_SIN2_RANGE[0]), sht._split_at(nside, RES_SIN2_RANGE[1])
     j = hi // ANA_BLOCK * ANA_BLOCK
-    return j if j > 0 and j >= lo else _split_at(nside, RES_SIN2_FALLBACK)
+    return j if j > 0 and j >= lo else sht._split_at(nside, RES_SIN2_FALLBACK)
 
 
 def _split_fields(nside, nact, Lt, jsplit):
@@ -121,7 +100,7 @@ def plan(nside, lmax, device=None, polar_skip=True):
     tab = sht.plan(nside, lmax + 2, 0, device, polar_skip)
     if nside >= ANA_BLOCK and int(_lib.query("gm_bat_blocks", nside, ANA_BLOCK + 1, 0)) != 2:
         raise RuntimeError("ANA_BLOCK does not match the library's analysis workgroup")
-    nact = _nactive_pairs(nside, lmax, polar_skip)
+    nact = sht._nactive_pairs(nside, lmax, polar_skip)
     Lt = lmax + 3  # table degrees
     jsplit, mpol, nb32, nb64, tsize64 = _split_fields(nside, nact, Lt, polar_split(nside))
     alpha = torch.zeros(tab.alpha.numel() + ALPHA_TAIL, dtype=torch.float64, device=device)

@@ -1,4 +1,5 @@
-// Latitudinal (Legendre / Wigner-d) stage of the HEALPix transforms on gfx950, FP64.
+// Latitudinal (Legendre / Wigner-d) stage of the HEALPix transforms on gfx950: spins other
+// than 0 and 2 in FP64, every spin in mixed precision (FP64 spin 0 and 2: pairs.hip).
 //
 // For each order m the normalised rows lambda_lm(theta) = sqrt((2l+1)/4pi) d^l_{m,-s}
 // are generated on the fly by the three-term recurrence in l, rescaled so that every
@@ -20,6 +21,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "pairs.h"
 #include "recurrence.h"
 
 namespace gm {
@@ -862,13 +864,11 @@ __global__ void k_prep_s(const double2* __restrict__ ae, const double2* __restri
 // ------------------------------------------------------------------ configs
 // Large geometries use 4-wave workgroups with R rings per lane, per precision and pass
 // (the mixed kernels hold half the registers per ring; the mixed syntheses keep their
-// accumulators in MFMA tiles).  Chosen by timing R = 3..10 on MI355X at Nside 4096:
+// accumulators in MFMA tiles).  The FP64 spin-0 kernels (pairs.hip) have shapes of their own;
+// here the FP64 spin-0 analysis only has its pass and slot counts.  Chosen by timing R = 3..10 on MI355X at Nside 4096:
 // occupancy steps make the best R differ between passes.
 #ifndef GM_ANA_R_S0
 #define GM_ANA_R_S0 6
-#endif
-#ifndef GM_SYN_R_S0
-#define GM_SYN_R_S0 4
 #endif
 #ifndef GM_ANA_R_S
 #define GM_ANA_R_S 8
@@ -894,7 +894,7 @@ __global__ void k_prep_s(const double2* __restrict__ ae, const double2* __restri
 constexpr int large_r(bool syn, bool mixed, bool spin0, int K = 1) {
     return (spin0 && K >= 8) ? 2
            : (spin0 && K >= 4) ? 3
-           : syn ? (mixed ? (spin0 ? GM_MIX_SYN_R_S0 : GM_MIX_SYN_R_S) : (spin0 ? GM_SYN_R_S0 : GM_SYN_R_S))
+           : syn ? (mixed ? (spin0 ? GM_MIX_SYN_R_S0 : GM_MIX_SYN_R_S) : GM_SYN_R_S)
                  : (mixed ? (spin0 ? GM_MIX_ANA_R_S0 : GM_MIX_ANA_R_S) : (spin0 ? GM_ANA_R_S0 : GM_ANA_R_S));
 }
 
@@ -986,31 +986,49 @@ extern "C" int gm_lat_tables(int64_t lmax, int64_t spin, double* alpha, double* 
 namespace gm {
 namespace {
 
-template <typename F>
-int launch_ana_s0(const char* name, const double* spec, int64_t nmaps, int64_t ld, int64_t smap, int64_t nside,
-                  int64_t lmax, const double* alpha, const double* seed_mant, const int32_t* seed_exp,
-                  const int32_t* nactive, double* partial, int64_t nchunks, int64_t chunk0, void* stream) {
+int check_s0(const char* name, bool mixed, bool pointers, int64_t nmaps, int64_t nside, int64_t lmax, int64_t ld,
+             int64_t smap) {
     if (int e = check_lat(nside, lmax, 0)) return e;
-    if (!spec || !alpha || !seed_mant || !seed_exp || !nactive || !partial) return fail(GM_E_ARG, "%s: null pointer", name);
-    constexpr bool mixed = std::is_same<F, float>::value;
+    if (!pointers) return fail(GM_E_ARG, "%s: null pointer", name);
     if (!(nmaps == 1 || nmaps == 2 || (mixed && (nmaps == 4 || nmaps == 8))))
         return fail(GM_E_ARG, mixed ? "%s: nmaps must be 1, 2, 4 or 8" : "%s: nmaps must be 1 or 2", name);
-    const int64_t L = lmax + 1;
-    if (ld < L) return fail(GM_E_SHAPE, "%s: ld < lmax + 1", name);
+    if (ld < lmax + 1) return fail(GM_E_SHAPE, "%s: ld < lmax + 1", name);
     if (nmaps > 1 && smap < (4 * nside - 1) * ld) return fail(GM_E_SHAPE, "%s: map stride too small", name);
-    const LatConfig cfg = lat_config(nside, 0, mixed, (int)nmaps);
+    return GM_OK;
+}
+
+int check_pass(const char* name, const LatConfig& cfg, int64_t nchunks, int64_t chunk0) {
     if (nchunks != cfg.nslots)
         return fail(GM_E_SHAPE, "%s: partial has %lld chunks, need %d", name, (long long)nchunks, cfg.nslots);
     if (chunk0 < 0 || chunk0 >= cfg.nchunks || chunk0 % cfg.nslots)
         return fail(GM_E_ARG, "%s: chunk0 %lld is not a pass start below %d", name, (long long)chunk0, cfg.nchunks);
+    return GM_OK;
+}
+
+// The ring pairs jbeg .. jend - 1 of an FP64 spin-0 pass (its chunks'), which the pair kernels
+// cover in slots of their own size.
+void pass_pairs(const LatConfig& cfg, int64_t nside, int64_t chunk0, int& jbeg, int& jend) {
+    const int64_t end = (chunk0 + cfg.nslots) * cfg.CH;
+    jbeg = (int)(chunk0 * cfg.CH);
+    jend = (int)(end < 2 * nside ? end : 2 * nside);
+}
+
+int launch_ana_s0_mixed(const char* name, const double* spec, int64_t nmaps, int64_t ld, int64_t smap, int64_t nside,
+                        int64_t lmax, const double* alpha, const double* seed_mant, const int32_t* seed_exp,
+                        const int32_t* nactive, double* partial, int64_t nchunks, int64_t chunk0, void* stream) {
+    const bool pointers = spec && alpha && seed_mant && seed_exp && nactive && partial;
+    if (int e = check_s0(name, true, pointers, nmaps, nside, lmax, ld, smap)) return e;
+    const int64_t L = lmax + 1;
+    const LatConfig cfg = lat_config(nside, 0, true, (int)nmaps);
+    if (int e = check_pass(name, cfg, nchunks, chunk0)) return e;
     const int64_t ts = table_size(L);
     const int nblk = cfg.nchunks - (int)chunk0 < cfg.nslots ? cfg.nchunks - (int)chunk0 : cfg.nslots;
     dim3 grid(nblk, (unsigned)L), block(64 * cfg.NW);
     hipStream_t st = (hipStream_t)stream;
     const double2* sp = reinterpret_cast<const double2*>(spec);
-    constexpr int RL = large_r(false, mixed, true);
-    if (int e = check_config(name, cfg, large_r(false, mixed, true, (int)nmaps))) return e;
-#define GM_ANA0(KK, RR, WW) hipLaunchKernelGGL((k_ana_s0<KK, RR, WW, F>), grid, block, 0, st, sp, ld, smap, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, partial, ts, (int)chunk0)
+    constexpr int RL = large_r(false, true, true);
+    if (int e = check_config(name, cfg, large_r(false, true, true, (int)nmaps))) return e;
+#define GM_ANA0(KK, RR, WW) hipLaunchKernelGGL((k_ana_s0<KK, RR, WW, float>), grid, block, 0, st, sp, ld, smap, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, partial, ts, (int)chunk0)
     if (nmaps == 1) {
         if (cfg.NW == 1) GM_ANA0(1, 2, 1);
         else if (cfg.NW == 2) GM_ANA0(1, 4, 2);
@@ -1019,16 +1037,14 @@ int launch_ana_s0(const char* name, const double* spec, int64_t nmaps, int64_t l
         if (cfg.NW == 1) GM_ANA0(2, 2, 1);
         else if (cfg.NW == 2) GM_ANA0(2, 4, 2);
         else GM_ANA0(2, RL, 4);
-    } else if constexpr (mixed) {
-        if (nmaps == 4) {
-            if (cfg.NW == 1) GM_ANA0(4, 2, 1);
-            else if (cfg.NW == 2) GM_ANA0(4, 4, 2);
-            else GM_ANA0(4, 3, 4);
-        } else {
-            if (cfg.NW == 1) GM_ANA0(8, 2, 1);
-            else if (cfg.NW == 2) GM_ANA0(8, 4, 2);
-            else GM_ANA0(8, 2, 4);
-        }
+    } else if (nmaps == 4) {
+        if (cfg.NW == 1) GM_ANA0(4, 2, 1);
+        else if (cfg.NW == 2) GM_ANA0(4, 4, 2);
+        else GM_ANA0(4, 3, 4);
+    } else {
+        if (cfg.NW == 1) GM_ANA0(8, 2, 1);
+        else if (cfg.NW == 2) GM_ANA0(8, 4, 2);
+        else GM_ANA0(8, 2, 4);
     }
 #undef GM_ANA0
     return check_launch(name);
@@ -1040,32 +1056,26 @@ int launch_ana_s0(const char* name, const double* spec, int64_t nmaps, int64_t l
 #define GM_MIX_SYN0_SINGLE_MFMA 1
 #endif
 
-template <typename F>
-int launch_syn_s0(const char* name, const double* coef, int64_t nmaps, int64_t nside, int64_t lmax, const double* alpha,
-                  const double* seed_mant, const int32_t* seed_exp, const int32_t* nactive, double* spec, int64_t ld,
-                  int64_t smap, void* stream) {
-    if (int e = check_lat(nside, lmax, 0)) return e;
-    if (!coef || !alpha || !seed_mant || !seed_exp || !nactive || !spec) return fail(GM_E_ARG, "%s: null pointer", name);
-    constexpr bool mixed = std::is_same<F, float>::value;
-    if (!(nmaps == 1 || nmaps == 2 || (mixed && (nmaps == 4 || nmaps == 8))))
-        return fail(GM_E_ARG, mixed ? "%s: nmaps must be 1, 2, 4 or 8" : "%s: nmaps must be 1 or 2", name);
+int launch_syn_s0_mixed(const char* name, const double* coef, int64_t nmaps, int64_t nside, int64_t lmax,
+                        const double* alpha, const double* seed_mant, const int32_t* seed_exp, const int32_t* nactive,
+                        double* spec, int64_t ld, int64_t smap, void* stream) {
+    const bool pointers = coef && alpha && seed_mant && seed_exp && nactive && spec;
+    if (int e = check_s0(name, true, pointers, nmaps, nside, lmax, ld, smap)) return e;
     const int64_t L = lmax + 1;
-    if (ld < L) return fail(GM_E_SHAPE, "%s: ld < lmax + 1", name);
-    if (nmaps > 1 && smap < (4 * nside - 1) * ld) return fail(GM_E_SHAPE, "%s: map stride too small", name);
-    const LatConfig cfg = syn_config(nside, 0, mixed, (int)nmaps);
+    const LatConfig cfg = syn_config(nside, 0, true, (int)nmaps);
     dim3 grid(cfg.nchunks, (unsigned)L), block(64 * cfg.NW);
     hipStream_t st = (hipStream_t)stream;
     const double2* cf = reinterpret_cast<const double2*>(coef);
     double2* sp = reinterpret_cast<double2*>(spec);
-    constexpr int RL = large_r(true, mixed, true);
-    if (int e = check_config(name, cfg, large_r(true, mixed, true, (int)nmaps))) return e;
+    constexpr int RL = large_r(true, true, true);
+    if (int e = check_config(name, cfg, large_r(true, true, true, (int)nmaps))) return e;
 #define GM_SYN0(KK, RR, WW)                                                                                       \
     do {                                                                                                          \
-        if constexpr (mixed && (KK > 1 || GM_MIX_SYN0_SINGLE_MFMA))                                               \
+        if constexpr (KK > 1 || GM_MIX_SYN0_SINGLE_MFMA)                                                          \
             hipLaunchKernelGGL((k_syn_s0_mx<KK, RR, WW>), grid, block, 0, st, cf, (int)nside, (int)L, alpha,      \
                                seed_mant, seed_exp, nactive, sp, ld, smap);                                        \
         else                                                                                                      \
-            hipLaunchKernelGGL((k_syn_s0<KK, RR, WW, F>), grid, block, 0, st, cf, (int)nside, (int)L, alpha,      \
+            hipLaunchKernelGGL((k_syn_s0<KK, RR, WW, float>), grid, block, 0, st, cf, (int)nside, (int)L, alpha,  \
                                seed_mant, seed_exp, nactive, sp, ld, smap);                                        \
     } while (0)
     if (nmaps == 1) {
@@ -1076,16 +1086,14 @@ int launch_syn_s0(const char* name, const double* coef, int64_t nmaps, int64_t n
         if (cfg.NW == 1) GM_SYN0(2, 2, 1);
         else if (cfg.NW == 2) GM_SYN0(2, 4, 2);
         else GM_SYN0(2, RL, 4);
-    } else if constexpr (mixed) {
-        if (nmaps == 4) {
-            if (cfg.NW == 1) GM_SYN0(4, 2, 1);
-            else if (cfg.NW == 2) GM_SYN0(4, 4, 2);
-            else GM_SYN0(4, 3, 4);
-        } else {
-            if (cfg.NW == 1) GM_SYN0(8, 2, 1);
-            else if (cfg.NW == 2) GM_SYN0(8, 4, 2);
-            else GM_SYN0(8, 2, 4);
-        }
+    } else if (nmaps == 4) {
+        if (cfg.NW == 1) GM_SYN0(4, 2, 1);
+        else if (cfg.NW == 2) GM_SYN0(4, 4, 2);
+        else GM_SYN0(4, 3, 4);
+    } else {
+        if (cfg.NW == 1) GM_SYN0(8, 2, 1);
+        else if (cfg.NW == 2) GM_SYN0(8, 4, 2);
+        else GM_SYN0(8, 2, 4);
     }
 #undef GM_SYN0
     return check_launch(name);
@@ -1161,16 +1169,25 @@ extern "C" int gm_lat_ana_s0(const double* spec, int64_t nmaps, int64_t ld, int6
                              int64_t lmax, const double* alpha, const double* seed_mant, const int32_t* seed_exp,
                              const int32_t* nactive, double* partial, int64_t nchunks, int64_t chunk0,
                              void* stream) {
-    return launch_ana_s0<double>("gm_lat_ana_s0", spec, nmaps, ld, smap, nside, lmax, alpha, seed_mant, seed_exp,
-                                 nactive, partial, nchunks, chunk0, stream);
+    const char* name = "gm_lat_ana_s0";
+    const bool pointers = spec && alpha && seed_mant && seed_exp && nactive && partial;
+    if (int e = check_s0(name, false, pointers, nmaps, nside, lmax, ld, smap)) return e;
+    const LatConfig cfg = lat_config(nside, 0);
+    if (int e = check_pass(name, cfg, nchunks, chunk0)) return e;
+    int jbeg, jend;
+    pass_pairs(cfg, nside, chunk0, jbeg, jend);
+    const int CH = pairs_chunk(nside, (int)nmaps), nblk = (jend - jbeg + CH - 1) / CH;
+    if (nblk > cfg.nslots) return fail(GM_E_LAUNCH, "%s: %d workgroups for %d partial slots", name, nblk, cfg.nslots);
+    return ana_pairs_s0(name, spec, (int)nmaps, ld, smap, nside, lmax + 1, alpha, seed_mant, seed_exp, nactive, partial,
+                        jbeg, jend, nblk, stream);
 }
 
 extern "C" int gm_lat_ana_s0_mixed(const double* spec, int64_t nmaps, int64_t ld, int64_t smap, int64_t nside,
                                    int64_t lmax, const double* alpha, const double* seed_mant, const int32_t* seed_exp,
                                    const int32_t* nactive, double* partial, int64_t nchunks, int64_t chunk0,
                                    void* stream) {
-    return launch_ana_s0<float>("gm_lat_ana_s0_mixed", spec, nmaps, ld, smap, nside, lmax, alpha, seed_mant, seed_exp,
-                                nactive, partial, nchunks, chunk0, stream);
+    return launch_ana_s0_mixed("gm_lat_ana_s0_mixed", spec, nmaps, ld, smap, nside, lmax, alpha, seed_mant, seed_exp,
+                               nactive, partial, nchunks, chunk0, stream);
 }
 
 namespace gm {
@@ -1186,6 +1203,12 @@ int finish_s0(const char* name, bool mixed, const double* partial, int64_t nmaps
     const int64_t L = lmax + 1, nelem = L * (L + 1) / 2;
     if (nmaps > 1 && alm_map_stride < nelem) return fail(GM_E_SHAPE, "%s: alm stride too small", name);
     const LatConfig cfg = lat_config(nside, 0, mixed, (int)nmaps);
+    if (!mixed) {
+        int jbeg, jend;
+        pass_pairs(cfg, nside, chunk0, jbeg, jend);
+        return finish_pairs_s0(name, partial, (int)nmaps, nside, L, nactive, P, alm, alm_map_stride, mode, jbeg, jend,
+                               stream);
+    }
     hipLaunchKernelGGL(k_finish_s0, dim3((unsigned)((L + 255) / 256), (unsigned)L), dim3(256), 0, (hipStream_t)stream,
                        reinterpret_cast<const double2*>(partial), (int)nmaps, cfg.nslots, cfg.CH, nactive, P, (int)L,
                        table_size(L), reinterpret_cast<double2*>(alm), alm_map_stride, mode, (int)chunk0);
@@ -1224,15 +1247,18 @@ extern "C" int gm_lat_prep_s0(const double* alm, int64_t nmaps, int64_t alm_map_
 extern "C" int gm_lat_syn_s0(const double* coef, int64_t nmaps, int64_t nside, int64_t lmax, const double* alpha,
                              const double* seed_mant, const int32_t* seed_exp, const int32_t* nactive, double* spec,
                              int64_t ld, int64_t smap, void* stream) {
-    return launch_syn_s0<double>("gm_lat_syn_s0", coef, nmaps, nside, lmax, alpha, seed_mant, seed_exp, nactive, spec,
-                                 ld, smap, stream);
+    const char* name = "gm_lat_syn_s0";
+    const bool pointers = coef && alpha && seed_mant && seed_exp && nactive && spec;
+    if (int e = check_s0(name, false, pointers, nmaps, nside, lmax, ld, smap)) return e;
+    return syn_pairs_s0(name, coef, (int)nmaps, nside, lmax + 1, alpha, seed_mant, seed_exp, nactive, spec, ld, smap,
+                        stream);
 }
 
 extern "C" int gm_lat_syn_s0_mixed(const double* coef, int64_t nmaps, int64_t nside, int64_t lmax, const double* alpha,
                                    const double* seed_mant, const int32_t* seed_exp, const int32_t* nactive,
                                    double* spec, int64_t ld, int64_t smap, void* stream) {
-    return launch_syn_s0<float>("gm_lat_syn_s0_mixed", coef, nmaps, nside, lmax, alpha, seed_mant, seed_exp, nactive,
-                                spec, ld, smap, stream);
+    return launch_syn_s0_mixed("gm_lat_syn_s0_mixed", coef, nmaps, nside, lmax, alpha, seed_mant, seed_exp, nactive,
+                               spec, ld, smap, stream);
 }
 
 extern "C" int gm_lat_ana_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, int64_t spin,

@@ -85,6 +85,28 @@ def _nactive(nside, lmax, spin, polar_skip):
     return np.searchsorted(-best, -m, side="right").astype(np.int32)
 
 
+def _nactive_pairs(nside, lmax, polar_skip):
+    """Ring pairs (equator first) that order m visits: the larger of ducc0's spin-0 and
+    spin-2 polar-skip bounds (``_nactive``), evaluated on the folded rings."""
+    z, sin = _ring_slots(nside, 0)
+    n = len(z)
+    L = lmax + 1
+    if not polar_skip:
+        return np.full(L, n, dtype=np.int32)
+    ofs = max(100.0, 0.01 * lmax)
+    b = lmax * sin + ofs
+    mlim0 = b
+    mlim2 = 2.0 * np.abs(z) + np.sqrt(np.maximum(b * b - 4.0 * sin * sin, 0.0))
+    best = np.maximum.accumulate(np.maximum(mlim0, mlim2)[::-1])[::-1]
+    return np.searchsorted(-best, -np.arange(L), side="right").astype(np.int32)
+
+
+def _split_at(nside, sin2):
+    """Number of ring pairs (from the equator) with sin^2(theta) >= sin2."""
+    _, sin = _ring_slots(nside, 0)
+    return int(np.count_nonzero(sin * sin >= sin2))
+
+
 @dataclass
 class Plan:
     nside: int
@@ -128,6 +150,54 @@ def plan(nside, lmax, spin, device=None, polar_skip=True):
         nchunks=int(_lib.query("gm_lat_nchunks", nside, spin)),
         tsize=tsize,
         nchunks_mixed=int(_lib.query("gm_lat_nchunks_mixed", nside, spin, 1)),
+    )
+    _PLANS[key] = p
+    return p
+
+
+# Ring pairs with sin^2(theta) below this run the spin-2 recurrence itself; the others the
+# spin-0 rows with weights 1/sin^2, which amplify rounding by up to this bound's inverse.
+PAIR_SIN2 = 1.0 / 32.0
+
+
+@dataclass
+class Plan2:
+    """FP64 spin-2 transforms on the spin-0 rows (``gm_lat2_*``)."""
+    nside: int
+    lmax: int
+    device: torch.device
+    tab: Plan              # spin-0 tables of lmax + 2
+    pol: Plan              # spin-2 tables (polar rings)
+    nact: torch.Tensor     # ring pairs visited by order m
+    jsplit: int            # first ring pair of the polar part
+    mpol: int              # orders that reach the polar rings
+    nslots: int
+    nchunks: int
+    nbp: int               # polar blocks per order
+    tsize: int             # entries of the spin-0 tables
+    ptsize: int            # entries of the spin-2 tables of the orders m < mpol
+
+
+def plan2(nside, lmax, device=None, polar_skip=True):
+    device = torch.device(device if device is not None else "cuda")
+    if device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    key = (int(nside), int(lmax), "pairs", device, bool(polar_skip))
+    p = _PLANS.get(key)
+    if p is not None:
+        return p
+    nside, lmax = int(nside), int(lmax)
+    L = lmax + 1
+    jsplit = _split_at(nside, PAIR_SIN2)
+    mpol = int(np.count_nonzero(_nactive(nside, lmax, 2, polar_skip) > 2 * jsplit - 1))
+    p = Plan2(
+        nside=nside, lmax=lmax, device=device, tab=plan(nside, lmax + 2, 0, device, polar_skip),
+        pol=plan(nside, lmax, 2, device, polar_skip),
+        nact=torch.as_tensor(_nactive_pairs(nside, lmax, polar_skip), dtype=torch.int32, device=device),
+        jsplit=jsplit, mpol=mpol, nslots=int(_lib.query("gm_lat2_slots", nside, jsplit)),
+        nchunks=int(_lib.query("gm_lat2_chunks", nside, jsplit)),
+        nbp=int(_lib.query("gm_lat2_polar_blocks", nside, jsplit)),
+        tsize=int(_lib.query("gm_table_size", lmax + 2)), ptsize=mpol * (L + 8) - mpol * (mpol - 1) // 2,
     )
     _PLANS[key] = p
     return p
@@ -333,6 +403,34 @@ def _synthesis_s(p, ae, ab, spec, mixed=False):
               _lib.ptr(p.smant), _lib.ptr(p.sexp), _lib.ptr(p.nact), _lib.ptr(spec), spec.shape[1], st)
 
 
+def _analysis_2(p, spec, ae, ab, mode):
+    """FP64 spin-2 analysis on the spin-0 rows (polar rings: the spin-2 recurrence)."""
+    st = _lib.stream_ptr(p.device)
+    part = torch.empty(p.nslots * p.tsize * 4, dtype=torch.float64, device=p.device)
+    ppart = torch.empty(p.nbp * p.ptsize * 4, dtype=torch.float64, device=p.device) if p.mpol else None
+    t, q = p.tab, p.pol
+    for c0 in range(0, p.nchunks, p.nslots):
+        md = int(mode) if c0 == 0 else (1 if mode == 1 else 2)
+        _lib.call("gm_lat2_ana", _lib.ptr(spec), spec.shape[1], p.nside, p.lmax, p.jsplit, p.mpol, _lib.ptr(t.alpha),
+                  _lib.ptr(t.smant), _lib.ptr(t.sexp), _lib.ptr(p.nact), _lib.ptr(q.alpha), _lib.ptr(q.gamma),
+                  _lib.ptr(q.smant), _lib.ptr(q.sexp), _lib.ptr(q.nact), _lib.ptr(part), _lib.ptr(ppart), c0, st)
+        _lib.call("gm_lat2_finish", _lib.ptr(part), _lib.ptr(ppart), p.nside, p.lmax, p.jsplit, p.mpol,
+                  _lib.ptr(p.nact), _lib.ptr(t.P), _lib.ptr(q.nact), _lib.ptr(q.P), _lib.ptr(ae), _lib.ptr(ab), md,
+                  c0, st)
+
+
+def _synthesis_2(p, ae, ab, spec):
+    st = _lib.stream_ptr(p.device)
+    coef = torch.empty(p.tsize * 2, dtype=torch.complex128, device=p.device)
+    pcoef = torch.empty(p.ptsize * 2, dtype=torch.complex128, device=p.device) if p.mpol else None
+    t, q = p.tab, p.pol
+    _lib.call("gm_lat2_prep", _lib.ptr(ae), _lib.ptr(ab), _lib.ptr(t.P), _lib.ptr(q.P), p.lmax, p.mpol, _lib.ptr(coef),
+              _lib.ptr(pcoef), st)
+    _lib.call("gm_lat2_syn", _lib.ptr(coef), _lib.ptr(pcoef), p.nside, p.lmax, p.jsplit, p.mpol, _lib.ptr(t.alpha),
+              _lib.ptr(t.smant), _lib.ptr(t.sexp), _lib.ptr(p.nact), _lib.ptr(q.alpha), _lib.ptr(q.gamma),
+              _lib.ptr(q.smant), _lib.ptr(q.sexp), _lib.ptr(q.nact), _lib.ptr(spec), spec.shape[1], st)
+
+
 def map2alm_spin(maps, lmax, spin, n_iter=0, polar_skip=True, precision="fp64"):
     """``(2, npix)`` (Q, U) -> ``(2, nelem)`` (E, B).  ``precision="mixed"`` as for spin 0."""
     maps = torch.as_tensor(maps)
@@ -344,7 +442,8 @@ def map2alm_spin(maps, lmax, spin, n_iter=0, polar_skip=True, precision="fp64"):
     nside = _check_nside(npix)
     lmax, spin = int(lmax), int(spin)
     _make_room(nside)
-    p = plan(nside, lmax, spin, dev, polar_skip)
+    pairs = spin == 2 and not _mixed(precision)
+    p = plan2(nside, lmax, dev, polar_skip) if pairs else plan(nside, lmax, spin, dev, polar_skip)
     L = lmax + 1
     W = 2 * L - 1
     nring = 4 * nside - 1
@@ -353,13 +452,19 @@ def map2alm_spin(maps, lmax, spin, n_iter=0, polar_skip=True, precision="fp64"):
     _lib.call("gm_ring_fft_fwd_s", _lib.ptr(maps[0]), _lib.ptr(maps[1]), nside, lmax, _lib.ptr(spec), W, st)
     nelem = L * (L + 1) // 2
     alm = torch.empty((2, nelem), dtype=torch.complex128, device=dev)
-    _analysis_s(p, spec, alm[0], alm[1], 0, _mixed(precision))
+
+    def ana(s_, a, mode, mx):
+        _analysis_2(p, s_, a[0], a[1], mode) if pairs else _analysis_s(p, s_, a[0], a[1], mode, mx)
+
+    def syn(a, s_, mx):
+        _synthesis_2(p, a[0], a[1], s_) if pairs else _synthesis_s(p, a[0], a[1], s_, mx)
+
+    ana(spec, alm, 0, _mixed(precision))
 
     def fold(f, g, out):
         _lib.call("gm_ring_fold_residual_c", _lib.ptr(f), _lib.ptr(g), _lib.ptr(out), W, nside, lmax, st)
 
-    return _refine(alm, n_iter, lambda s_, a, mode, mx: _analysis_s(p, s_, a[0], a[1], mode, mx),
-                   lambda a, s_, mx: _synthesis_s(p, a[0], a[1], s_, mx), fold, spec, _mixed(precision))
+    return _refine(alm, n_iter, ana, syn, fold, spec, _mixed(precision))
 
 
 def alm2map_spin(alm, nside, lmax, spin, polar_skip=True, precision="fp64"):
@@ -370,11 +475,13 @@ def alm2map_spin(alm, nside, lmax, spin, polar_skip=True, precision="fp64"):
     L = lmax + 1
     if alm.ndim != 2 or alm.shape != (2, L * (L + 1) // 2):
         raise ValueError("Input alm has wrong shape")
-    p = plan(nside, lmax, spin, dev, polar_skip)
     W = 2 * L - 1
     nring = 4 * nside - 1
     spec = torch.empty((nring, W), dtype=torch.complex128, device=dev)
-    _synthesis_s(p, alm[0], alm[1], spec, _mixed(precision))
+    if spin == 2 and not _mixed(precision):
+        _synthesis_2(plan2(nside, lmax, dev, polar_skip), alm[0], alm[1], spec)
+    else:
+        _synthesis_s(plan(nside, lmax, spin, dev, polar_skip), alm[0], alm[1], spec, _mixed(precision))
     npix = 12 * nside * nside
     maps = torch.empty((2, npix), dtype=torch.float64, device=dev)
     _lib.call("gm_ring_fft_inv_s", _lib.ptr(spec), W, nside, lmax, _lib.ptr(maps[0]), _lib.ptr(maps[1]),
