@@ -25,6 +25,10 @@ SIGNATURES = {
     "gm_ring_fft_fwd_s": [_p, _p, _i64, _i64, _p, _i64, _p],
     "gm_ring_fft_inv_s0": [_p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p],
     "gm_ring_fft_inv_s": [_p, _i64, _i64, _i64, _p, _p, _p],
+    "gm_ring_pair_fwd_s0": [_p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _p],
+    "gm_ring_pair_fwd_s": [_p, _p, _i64, _i64, _p, _i64, _p],
+    "gm_ring_pair_inv_s0": [_p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p],
+    "gm_ring_pair_inv_s": [_p, _i64, _i64, _i64, _p, _p, _p],
     "gm_ring_fold_residual": [_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p],
     "gm_ring_fold_residual_c": [_p, _p, _p, _i64, _i64, _i64, _p],
     "gm_lat_tables": [_i64, _i64, _p, _p, _p, _p],

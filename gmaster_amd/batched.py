@@ -286,10 +286,10 @@ def alm2map(alm0, alm2, nside, lmax, polar_skip=True, out=None):
         _check_out(out[1], (k2, 2, npix), torch.float64, dev)
     if k0:
         maps0 = out[0] if out is not None else torch.empty((k0, npix), dtype=torch.float64, device=dev)
-        _lib.call("gm_ring_fft_inv_s0", _lib.ptr(spec0), k0, L, spec0.stride(0), nside, lmax, _lib.ptr(maps0), npix, st)
+        _lib.call("gm_ring_pair_inv_s0", _lib.ptr(spec0), k0, L, spec0.stride(0), nside, lmax, _lib.ptr(maps0), npix, st)
     if k2:
         maps2 = out[1] if out is not None else torch.empty((k2, 2, npix), dtype=torch.float64, device=dev)
         for f in range(k2):
-            _lib.call("gm_ring_fft_inv_s", _lib.ptr(spec2[f]), W, nside, lmax, _lib.ptr(maps2[f, 0]),
+            _lib.call("gm_ring_pair_inv_s", _lib.ptr(spec2[f]), W, nside, lmax, _lib.ptr(maps2[f, 0]),
                       _lib.ptr(maps2[f, 1]), st)
     return maps0, maps2

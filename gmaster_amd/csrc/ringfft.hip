@@ -7,6 +7,12 @@
 // output per thread) for larger prime factors.  One workgroup per ring; rings are
 // launched in size buckets so the dynamic LDS matches the largest ring of the bucket.
 //
+// gm_ring_pair_* take caps up to q = 2048 and the belts of Nside 64 .. 2048 two rings at a time
+// (ringpair.hip) and the other rings here; gm_ring_fft_* take every ring here.  The fast forms
+// call the latter ahead of their 16-bit operand splits: another FP64 rounding of a spectrum
+// (1e-15) moves some splits by a unit, 7e-9 of the alms at Nside 512, and their results are to
+// stay what they were.
+//
 // The forward output is the *phased* spectrum  G[r][m] = w e^{-i m phi0} X[m mod n]
 // (w = 4 pi / npix), exactly the right-hand side of the Legendre analysis, so no
 // separate weight / phase pass runs.  The Jacobi residual is formed in this space by
@@ -18,6 +24,7 @@
 #include <vector>
 
 #include "common.h"
+#include "ringpair.h"
 
 namespace gm {
 
@@ -1033,11 +1040,11 @@ struct Bucket {
 
 // Size buckets: the small caps together (N = 2q <= 512: one launch instead of one per
 // power of two, each of which would hold a handful of workgroups), then caps with
-// N = 2q in (2^(b-1), 2^b], then the belt.
-int make_buckets(int nside, Bucket* out) {
+// N = 2q in (2^(b-1), 2^b], then the belt; with pairs, without what the pair transforms take.
+int make_buckets(int nside, bool pairs, Bucket* out) {
     int nb = 0;
-    int q = 1;
-    if (nside - 1 >= 1) {
+    int q = pairs ? kRingPairQ + 1 : 1;
+    if (nside - 1 >= 1 && !pairs) {
         const int qhi = nside - 1 < 256 ? nside - 1 : 256;
         out[nb].qlo = 1;
         out[nb].qhi = qhi;
@@ -1059,6 +1066,7 @@ int make_buckets(int nside, Bucket* out) {
         ++nb;
         q = qhi + 1;
     }
+    if (pairs && ring_pair_belt(nside)) return nb;
     out[nb].qlo = 0;
     out[nb].qhi = 0;
     out[nb].nblocks = 2 * nside + 1;
@@ -1100,6 +1108,19 @@ inline size_t table_bytes(int dcap) { return (size_t)(dcap / 8 + 1) * sizeof(dou
 // launched no other runtime call is made (HIP graph capture records launches only).
 template <typename K>
 int set_lds(K kernel, size_t bytes) {
+    return ring_set_lds(reinterpret_cast<const void*>(kernel), bytes);
+}
+
+int check_ring_args(int64_t nside, int64_t lmax) {
+    if (nside < 1 || (nside & (nside - 1)) != 0) return fail(GM_E_ARG, "nside must be a power of 2 (got %lld)", (long long)nside);
+    if (nside > kMaxNside) return fail(GM_E_UNSUPPORTED, "ring FFT supports nside <= %d (got %lld)", kMaxNside, (long long)nside);
+    if (lmax < 0) return fail(GM_E_ARG, "lmax must be >= 0");
+    return GM_OK;
+}
+
+}  // namespace
+
+int ring_set_lds(const void* fn, size_t bytes) {
     if (bytes <= 64 * 1024) return GM_OK;
     constexpr size_t kBase = (size_t)kLdsN * sizeof(double2);
     int dev = 0;
@@ -1111,7 +1132,6 @@ int set_lds(K kernel, size_t bytes) {
         size_t bytes;
     };
     static std::vector<Limit> done;
-    const void* fn = reinterpret_cast<const void*>(kernel);
     std::lock_guard<std::mutex> lock(mu);
     Limit* cur = nullptr;
     for (auto& d : done)
@@ -1127,22 +1147,14 @@ int set_lds(K kernel, size_t bytes) {
     return GM_OK;
 }
 
-int check_ring_args(int64_t nside, int64_t lmax) {
-    if (nside < 1 || (nside & (nside - 1)) != 0) return fail(GM_E_ARG, "nside must be a power of 2 (got %lld)", (long long)nside);
-    if (nside > kMaxNside) return fail(GM_E_UNSUPPORTED, "ring FFT supports nside <= %d (got %lld)", kMaxNside, (long long)nside);
-    if (lmax < 0) return fail(GM_E_ARG, "lmax must be >= 0");
-    return GM_OK;
-}
-
-}  // namespace
-
 }  // namespace gm
 
 using namespace gm;
 
-extern "C" int gm_ring_fft_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside,
-                                  int64_t lmax, double* spec, int64_t ld, int64_t spec_map_stride,
-                                  void* stream) {
+namespace {
+
+int ring_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside, int64_t lmax, double* spec,
+                int64_t ld, int64_t spec_map_stride, void* stream, bool pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
     if (!maps || !spec) return fail(GM_E_ARG, "gm_ring_fft_fwd_s0: null pointer");
     const int64_t L = lmax + 1, npix = 12 * nside * nside, nring = 4 * nside - 1;
@@ -1150,8 +1162,13 @@ extern "C" int gm_ring_fft_fwd_s0(const double* maps, int64_t nmaps, int64_t map
     if (ld < L) return fail(GM_E_SHAPE, "gm_ring_fft_fwd_s0: ld (%lld) < lmax + 1", (long long)ld);
     if (nmaps > 1 && (map_stride < npix || spec_map_stride < nring * ld))
         return fail(GM_E_SHAPE, "gm_ring_fft_fwd_s0: map strides too small");
+    if (pairs) {
+        const RingArgs ra{maps, nullptr, map_stride, (int)nmaps, (int)nside, (int)L, reinterpret_cast<double2*>(spec),
+                          ld, spec_map_stride, (hipStream_t)stream};
+        if (int e = ring_pairs_fwd(ra, false)) return e;
+    }
     Bucket b[32];
-    const int nb = make_buckets((int)nside, b);
+    const int nb = make_buckets((int)nside, pairs, b);
     for (int i = 0; i < nb; ++i) {
         const bool split = b[i].N > kLdsN;
         const int NL = split ? b[i].N / 2 : b[i].N;  // points held in LDS
@@ -1178,14 +1195,19 @@ extern "C" int gm_ring_fft_fwd_s0(const double* maps, int64_t nmaps, int64_t map
     return check_launch("gm_ring_fft_fwd_s0");
 }
 
-extern "C" int gm_ring_fft_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec,
-                                 int64_t ld, void* stream) {
+int ring_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec, int64_t ld, void* stream,
+               bool pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
     if (!q || !u || !spec) return fail(GM_E_ARG, "gm_ring_fft_fwd_s: null pointer");
     const int64_t L = lmax + 1;
     if (ld < 2 * L - 1) return fail(GM_E_SHAPE, "gm_ring_fft_fwd_s: ld (%lld) < 2 lmax + 1", (long long)ld);
+    if (pairs) {
+        const RingArgs ra{q, u, 0, 1, (int)nside, (int)L, reinterpret_cast<double2*>(spec), ld, 0,
+                          (hipStream_t)stream};
+        if (int e = ring_pairs_fwd(ra, true)) return e;
+    }
     Bucket b[32];
-    const int nb = make_buckets((int)nside, b);
+    const int nb = make_buckets((int)nside, pairs, b);
     for (int i = 0; i < nb; ++i) {
         const bool split = b[i].N > kLdsN;
         const int NL = split ? b[i].N / 2 : b[i].N;  // points held in LDS
@@ -1212,8 +1234,8 @@ extern "C" int gm_ring_fft_fwd_s(const double* q, const double* u, int64_t nside
     return check_launch("gm_ring_fft_fwd_s");
 }
 
-extern "C" int gm_ring_fft_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride,
-                                  int64_t nside, int64_t lmax, double* maps, int64_t map_stride, void* stream) {
+int ring_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride, int64_t nside, int64_t lmax,
+                double* maps, int64_t map_stride, void* stream, bool pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
     if (!maps || !spec) return fail(GM_E_ARG, "gm_ring_fft_inv_s0: null pointer");
     const int64_t L = lmax + 1, npix = 12 * nside * nside, nring = 4 * nside - 1;
@@ -1221,8 +1243,14 @@ extern "C" int gm_ring_fft_inv_s0(const double* spec, int64_t nmaps, int64_t ld,
     if (ld < L) return fail(GM_E_SHAPE, "gm_ring_fft_inv_s0: ld < lmax + 1");
     if (nmaps > 1 && (map_stride < npix || spec_map_stride < nring * ld))
         return fail(GM_E_SHAPE, "gm_ring_fft_inv_s0: map strides too small");
+    if (pairs) {
+        const RingArgs ra{maps, nullptr, map_stride, (int)nmaps, (int)nside, (int)L,
+                          reinterpret_cast<double2*>(const_cast<double*>(spec)), ld, spec_map_stride,
+                          (hipStream_t)stream};
+        if (int e = ring_pairs_inv(ra, false)) return e;
+    }
     Bucket b[32];
-    const int nb = make_buckets((int)nside, b);
+    const int nb = make_buckets((int)nside, pairs, b);
     for (int i = 0; i < nb; ++i) {
         const bool split = b[i].N > kLdsN;
         const int NL = split ? b[i].N / 2 : b[i].N;  // points held in LDS
@@ -1249,14 +1277,19 @@ extern "C" int gm_ring_fft_inv_s0(const double* spec, int64_t nmaps, int64_t ld,
     return check_launch("gm_ring_fft_inv_s0");
 }
 
-extern "C" int gm_ring_fft_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q,
-                                 double* u, void* stream) {
+int ring_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q, double* u, void* stream, bool
+               pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
     if (!spec || !q || !u) return fail(GM_E_ARG, "gm_ring_fft_inv_s: null pointer");
     const int64_t L = lmax + 1;
     if (ld < 2 * L - 1) return fail(GM_E_SHAPE, "gm_ring_fft_inv_s: ld < 2 lmax + 1");
+    if (pairs) {
+        const RingArgs ra{q, u, 0, 1, (int)nside, (int)L, reinterpret_cast<double2*>(const_cast<double*>(spec)), ld,
+                          0, (hipStream_t)stream};
+        if (int e = ring_pairs_inv(ra, true)) return e;
+    }
     Bucket b[32];
-    const int nb = make_buckets((int)nside, b);
+    const int nb = make_buckets((int)nside, pairs, b);
     for (int i = 0; i < nb; ++i) {
         const bool split = b[i].N > kLdsN;
         const int NL = split ? b[i].N / 2 : b[i].N;  // points held in LDS
@@ -1281,6 +1314,48 @@ extern "C" int gm_ring_fft_inv_s(const double* spec, int64_t ld, int64_t nside, 
         }
     }
     return check_launch("gm_ring_fft_inv_s");
+}
+
+}  // namespace
+
+extern "C" int gm_ring_fft_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside, int64_t lmax,
+                                  double* spec, int64_t ld, int64_t spec_map_stride, void* stream) {
+    return ring_fwd_s0(maps, nmaps, map_stride, nside, lmax, spec, ld, spec_map_stride, stream, false);
+}
+
+extern "C" int gm_ring_pair_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside, int64_t lmax,
+                                   double* spec, int64_t ld, int64_t spec_map_stride, void* stream) {
+    return ring_fwd_s0(maps, nmaps, map_stride, nside, lmax, spec, ld, spec_map_stride, stream, true);
+}
+
+extern "C" int gm_ring_fft_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec, int64_t
+                                 ld, void* stream) {
+    return ring_fwd_s(q, u, nside, lmax, spec, ld, stream, false);
+}
+
+extern "C" int gm_ring_pair_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec, int64_t
+                                  ld, void* stream) {
+    return ring_fwd_s(q, u, nside, lmax, spec, ld, stream, true);
+}
+
+extern "C" int gm_ring_fft_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride, int64_t
+                                  nside, int64_t lmax, double* maps, int64_t map_stride, void* stream) {
+    return ring_inv_s0(spec, nmaps, ld, spec_map_stride, nside, lmax, maps, map_stride, stream, false);
+}
+
+extern "C" int gm_ring_pair_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride, int64_t
+                                   nside, int64_t lmax, double* maps, int64_t map_stride, void* stream) {
+    return ring_inv_s0(spec, nmaps, ld, spec_map_stride, nside, lmax, maps, map_stride, stream, true);
+}
+
+extern "C" int gm_ring_fft_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q, double* u,
+                                 void* stream) {
+    return ring_inv_s(spec, ld, nside, lmax, q, u, stream, false);
+}
+
+extern "C" int gm_ring_pair_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q, double* u,
+                                  void* stream) {
+    return ring_inv_s(spec, ld, nside, lmax, q, u, stream, true);
 }
 
 extern "C" int gm_ring_fold_residual(const double* F, const double* G, double* R, int64_t nmaps, int64_t ld,

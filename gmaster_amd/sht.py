@@ -5,7 +5,8 @@ share one latitudinal pass, e.g. a field and its mask) and spin s (Q, U -> E, B)
 
 Pipeline of one analysis (``gmaster/_sht/healpix.py:1741-1926`` is the reference router):
 
-1. ring FFT of every ring into the phased spectrum ``G[r][m]`` (kernel ``gm_ring_fft_fwd_*``);
+1. ring FFT of every ring into the phased spectrum ``G[r][m]`` (kernel ``gm_ring_pair_fwd_*``,
+   in the fast form ``gm_ring_fft_fwd_*``);
 2. Legendre / Wigner-d analysis per order m over all rings (``gm_lat_ana_*``), then a
    finish kernel that sums the ring chunks, applies the per-(l, m) scale and (spin s)
    combines +-m into E/B;
@@ -337,7 +338,8 @@ def map2alm_s0(maps, lmax, n_iter=0, polar_skip=True, precision="fp64", max_grou
     nring = 4 * nside - 1
     st = _lib.stream_ptr(dev)
     spec = torch.empty((K, nring, L), dtype=torch.complex128, device=dev)
-    _lib.call("gm_ring_fft_fwd_s0", _lib.ptr(maps), K, npix, nside, lmax, _lib.ptr(spec), L, spec.stride(0), st)
+    _lib.call(_ring_fft("fwd_s0", precision), _lib.ptr(maps), K, npix, nside, lmax, _lib.ptr(spec), L,
+              spec.stride(0), st)
     nelem = L * (L + 1) // 2
     alm = torch.empty((K, nelem), dtype=torch.complex128, device=dev)
     _analysis_s0(p, spec, alm, 0, _mixed(precision))
@@ -354,6 +356,12 @@ def _mixed(precision):
     if precision not in ("fp64", "mixed"):
         raise ValueError("precision must be 'fp64' or 'mixed'")
     return precision == "mixed"
+
+
+def _ring_fft(name, precision):
+    """Ring FFT entry of a form: pairs of rings for FP64; ring by ring for the fast form, whose
+    operand splits would turn the last bit of a spectrum into 1e-8 of the alms."""
+    return ("gm_ring_fft_" if _mixed(precision) else "gm_ring_pair_") + name
 
 
 def alm2map_s0(alm, nside, lmax, polar_skip=True, precision="fp64", max_group=2):
@@ -375,7 +383,7 @@ def alm2map_s0(alm, nside, lmax, polar_skip=True, precision="fp64", max_group=2)
     _synthesis_s0(p, alm, spec, _mixed(precision))
     npix = 12 * nside * nside
     maps = torch.empty((K, npix), dtype=torch.float64, device=dev)
-    _lib.call("gm_ring_fft_inv_s0", _lib.ptr(spec), K, L, spec.stride(0), nside, lmax, _lib.ptr(maps), npix,
+    _lib.call(_ring_fft("inv_s0", precision), _lib.ptr(spec), K, L, spec.stride(0), nside, lmax, _lib.ptr(maps), npix,
               _lib.stream_ptr(dev))
     return maps
 
@@ -449,7 +457,7 @@ def map2alm_spin(maps, lmax, spin, n_iter=0, polar_skip=True, precision="fp64"):
     nring = 4 * nside - 1
     st = _lib.stream_ptr(dev)
     spec = torch.empty((nring, W), dtype=torch.complex128, device=dev)
-    _lib.call("gm_ring_fft_fwd_s", _lib.ptr(maps[0]), _lib.ptr(maps[1]), nside, lmax, _lib.ptr(spec), W, st)
+    _lib.call(_ring_fft("fwd_s", precision), _lib.ptr(maps[0]), _lib.ptr(maps[1]), nside, lmax, _lib.ptr(spec), W, st)
     nelem = L * (L + 1) // 2
     alm = torch.empty((2, nelem), dtype=torch.complex128, device=dev)
 
@@ -484,7 +492,7 @@ def alm2map_spin(alm, nside, lmax, spin, polar_skip=True, precision="fp64"):
         _synthesis_s(plan(nside, lmax, spin, dev, polar_skip), alm[0], alm[1], spec, _mixed(precision))
     npix = 12 * nside * nside
     maps = torch.empty((2, npix), dtype=torch.float64, device=dev)
-    _lib.call("gm_ring_fft_inv_s", _lib.ptr(spec), W, nside, lmax, _lib.ptr(maps[0]), _lib.ptr(maps[1]),
+    _lib.call(_ring_fft("inv_s", precision), _lib.ptr(spec), W, nside, lmax, _lib.ptr(maps[0]), _lib.ptr(maps[1]),
               _lib.stream_ptr(dev))
     return maps
 

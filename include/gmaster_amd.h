@@ -72,6 +72,17 @@ int gm_ring_fft_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t sp
 int gm_ring_fft_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q,
                       double* u, void* stream);
 
+/* The same four with rings taken in pairs up to Nside 2048 (as fast or faster; the values agree
+ * with those above to FP64 rounding). */
+int gm_ring_pair_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside,
+                        int64_t lmax, double* spec, int64_t ld, int64_t spec_map_stride, void* stream);
+int gm_ring_pair_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec,
+                       int64_t ld, void* stream);
+int gm_ring_pair_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride,
+                        int64_t nside, int64_t lmax, double* maps, int64_t map_stride, void* stream);
+int gm_ring_pair_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q,
+                       double* u, void* stream);
+
 /* Jacobi residual in ring-Fourier space, no FFT:
  *   R[r][k] = w nphi sum_{m = k mod nphi, |m| < L} e^{i (m-k) phi0} F[r][m] - G[r][k]
  * (spin 0: F[-m] = conj F[m]).  In-place allowed (R == G).
