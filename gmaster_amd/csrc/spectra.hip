@@ -10,28 +10,46 @@ namespace {
 constexpr int kClMChunk = 32;  // orders per partial in the coupled-C_ell reduction
 
 // partial[mc][pair][l] = sum_{m in chunk mc, m <= l} c_m Re(a_lm conj b_lm)
-__global__ void k_cl_partial(const double2* __restrict__ a, int n1, const double2* __restrict__ b, int n2,
-                             int64_t stride, int L, double* __restrict__ part) {
+// Bound: HBM for large lmax, else latency: the loads of kClStep orders are in flight together (one
+// order at a time behind run-time component loops before: 24 us for 2 x 2 components at
+// lmax 767, now 8 us).  Orders past l read order l and are dropped.
+constexpr int kClStep = 8;
+
+template <int N1, int N2>
+__global__ __launch_bounds__(256) void k_cl_partial(const double2* __restrict__ a, const double2* __restrict__ b,
+                                                    int64_t stride, int L, double* __restrict__ part) {
     const int l = blockIdx.x * blockDim.x + threadIdx.x;
     const int mc = blockIdx.y;
     const int m0 = mc * kClMChunk;
     if (l >= L || m0 > l) return;
-    const int mend = min(m0 + kClMChunk, l + 1);
     const int lmax = L - 1;
-    const int np = n1 * n2;
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int m = m0; m < mend; ++m) {
-        const int64_t ia = alm_index(l, m, lmax);
-        const double w = m ? 2.0 : 1.0;
-        for (int i = 0; i < n1; ++i) {
-            const double2 x = a[i * stride + ia];
-            for (int j = 0; j < n2; ++j) {
-                const double2 y = b[j * stride + ia];
-                acc[i * n2 + j] += w * (x.x * y.x + x.y * y.y);
+    double acc[N1 * N2];
+#pragma unroll
+    for (int p = 0; p < N1 * N2; ++p) acc[p] = 0.0;
+    for (int ms = m0; ms < min(m0 + kClMChunk, l + 1); ms += kClStep) {
+        double2 x[kClStep][N1], y[kClStep][N2];
+#pragma unroll
+        for (int u = 0; u < kClStep; ++u) {
+            const int64_t ia = alm_index(l, min(ms + u, l), lmax);
+#pragma unroll
+            for (int i = 0; i < N1; ++i) x[u][i] = a[i * stride + ia];
+#pragma unroll
+            for (int j = 0; j < N2; ++j) y[u][j] = b[j * stride + ia];
+        }
+#pragma unroll
+        for (int u = 0; u < kClStep; ++u) {
+            const double w = ms + u ? 2.0 : 1.0;
+            if (ms + u <= l) {
+#pragma unroll
+                for (int i = 0; i < N1; ++i)
+#pragma unroll
+                    for (int j = 0; j < N2; ++j)
+                        acc[i * N2 + j] += w * (x[u][i].x * y[u][j].x + x[u][i].y * y[u][j].y);
             }
         }
     }
-    for (int p = 0; p < np; ++p) part[((int64_t)mc * np + p) * L + l] = acc[p];
+#pragma unroll
+    for (int p = 0; p < N1 * N2; ++p) part[((int64_t)mc * (N1 * N2) + p) * L + l] = acc[p];
 }
 
 __global__ void k_cl_final(const double* __restrict__ part, int np, int L, double* __restrict__ cl) {
@@ -40,7 +58,14 @@ __global__ void k_cl_final(const double* __restrict__ part, int np, int L, doubl
     if (l >= L) return;
     const int nmc = l / kClMChunk + 1;
     double s = 0.0;
-    for (int mc = 0; mc < nmc; ++mc) s += part[((int64_t)mc * np + p) * L + l];
+    for (int ms = 0; ms < nmc; ms += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = part[((int64_t)min(ms + u, nmc - 1) * np + p) * L + l];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (ms + u < nmc) s += v[u];
+    }
     cl[(int64_t)p * L + l] = s / (2.0 * l + 1.0);
 }
 
@@ -55,7 +80,11 @@ __global__ void k_bin_cell(const double* __restrict__ cl, int64_t ld, const int*
     out[(int64_t)c * nb + b] = s;
 }
 
-// out[b1][b2] = sum_{e1 in b1, e2 in b2} wout[e1] M[ells[e1]][ells[e2]] tin[e2]
+// out[b1][b2] = sum_{e1 in b1, e2 in b2} wout[e1] M[ells[e1]][ells[e2]] tin[e2].  Bound: latency of
+// the matrix's words (one row after the other before: 115 us for a 3072 x 3072 block, 4 degrees a
+// bin; kBinRows rows together: 64 us).
+constexpr int kBinRows = 4;
+
 __global__ void k_bin_block(const double* __restrict__ M, int L, const int* __restrict__ ells,
                             const int* __restrict__ bstart, int nb, const double* __restrict__ wout,
                             const double* __restrict__ tin, double* __restrict__ out) {
@@ -63,11 +92,24 @@ __global__ void k_bin_block(const double* __restrict__ M, int L, const int* __re
     const int b1 = blockIdx.y;
     if (b2 >= nb) return;
     double s = 0.0;
-    for (int e1 = bstart[b1]; e1 < bstart[b1 + 1]; ++e1) {
-        const double* row = M + (int64_t)ells[e1] * L;
-        double r = 0.0;
-        for (int e2 = bstart[b2]; e2 < bstart[b2 + 1]; ++e2) r += row[ells[e2]] * tin[e2];
-        s += wout[e1] * r;
+    const int end = bstart[b1 + 1];
+    for (int e1 = bstart[b1]; e1 < end; e1 += kBinRows) {
+        const double* row[kBinRows];
+        double r[kBinRows];
+#pragma unroll
+        for (int u = 0; u < kBinRows; ++u) {
+            row[u] = M + (int64_t)ells[min(e1 + u, end - 1)] * L;
+            r[u] = 0.0;
+        }
+        for (int e2 = bstart[b2]; e2 < bstart[b2 + 1]; ++e2) {
+            const int c = ells[e2];
+            const double t = tin[e2];
+#pragma unroll
+            for (int u = 0; u < kBinRows; ++u) r[u] += row[u][c] * t;
+        }
+#pragma unroll
+        for (int u = 0; u < kBinRows; ++u)
+            if (e1 + u < end) s += wout[e1 + u] * r[u];
     }
     out[(int64_t)b1 * nb + b2] = s;
 }
@@ -92,9 +134,11 @@ extern "C" int gm_coupled_cell(const double* alm1, int64_t n1, const double* alm
     const int nmc = (int)((L + kClMChunk - 1) / kClMChunk);
     const int np = (int)(n1 * n2);
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_cl_partial, dim3((unsigned)((L + 255) / 256), nmc), dim3(256), 0, st,
-                       reinterpret_cast<const double2*>(alm1), (int)n1, reinterpret_cast<const double2*>(alm2),
-                       (int)n2, alm_stride, (int)L, work);
+    const auto kernel = n1 == 1 ? (n2 == 1 ? &k_cl_partial<1, 1> : &k_cl_partial<1, 2>)
+                                : (n2 == 1 ? &k_cl_partial<2, 1> : &k_cl_partial<2, 2>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((L + 255) / 256), nmc), dim3(256), 0, st,
+                       reinterpret_cast<const double2*>(alm1), reinterpret_cast<const double2*>(alm2), alm_stride,
+                       (int)L, work);
     hipLaunchKernelGGL(k_cl_final, dim3((unsigned)((L + 255) / 256), np), dim3(256), 0, st, work, np, (int)L, cl);
     return check_launch("gm_coupled_cell");
 }
