@@ -1,25 +1,25 @@
-// The l3 recursion of the mode-coupling row sums for one pair l1 <= l2, without square
+// The row sums of the mode-coupling matrix for one pair l1 <= l2, walked in l3 without square
 // roots (host and device).
 //
-// Both Wigner rows f0 = (l1 l2 l3; 0 0 0) and f2 = (l1 l2 l3; 2 -2 0) obey, for m3 = 0,
-//     Q(l3+1) f(l3+1) = c(l3) f(l3) - Q(l3) f(l3-1),
+// f0 = (l1 l2 l3; 0 0 0) obeys Q(l3+1) f0(l3+1) = -Q(l3) f0(l3-1) with
 //     Q(l3)^2 = q(l3) = (l3^2 - d^2) ((l1+l2+1)^2 - l3^2),   d = l2 - l1,
-// with c = 4 (2 l3 + 1) for f2 and c = 0 for f0, started from the closed forms at l3 = d
-// and run forward (stable for |m| <= 2 up to l3 = l1 + l2).  Scaled by
-// pi(l3) = Q(d+1) ... Q(l3), the values F = f pi obey
-//     F(l3+1) = c(l3) F(l3) - q(l3) F(l3-1),
-// which needs only the integer products q, so no square root or division per step.  The
-// sums sum_l3 W'_l3 f^2 = sum W' F^2 / pi^2 are accumulated in Horner form,
-// G <- G * (pi_new / pi_old)^2 + W' F^2, with pi^2 tracked as P (every even and every odd
-// degree has its own chain: the 0-0, 0-2 and 2-2+ sums take even J = l1 + l2 + l3, the
-// 2-2- sum odd J), and divided out once at the end.  P grows by at most S^4 / 4 < 2^57
-// per degree (S = l1 + l2 + 1 < 2^15); every 4 pairs of degrees F, P and G are rescaled
-// by powers of two (exact), so nothing leaves the FP64 range.
+// from the closed form at l3 = d, so f0^2 at even J = l1 + l2 + l3 (l3 = d, d + 2, ...) is R / P
+// with R the product of q over the odd degrees passed and P over the even ones.
 //
-// d = 0: the unnormalised recursion (Schulten-Gordon) is empty at l3 = 0, but the step
-// F2(1) = c(0) F2(0) = 4 f2(0) is still right: with (l l 0; 2 -2 0) = (-1)^l / sqrt(2l+1),
-// (l l 1; 2 -2 0) = (-1)^l 2 / sqrt(l (l+1)(2l+1)) and Q(1) = sqrt((2l+1)^2 - 1), both sides
-// equal 4 (-1)^l / sqrt(2l+1).
+// f2 = (l1 l2 l3; 2 -2 0) needs no recursion of its own.  The m recursion of 3j symbols
+// (Schulten & Gordon 1975), (L1 + L2 - 2 m^2 - X) f_m + C(m+1) f_{m+1} + C(m) f_{m-1} = 0 with
+// X = l3 (l3+1), L = l (l+1) and f_{-1} = f_1 at even J, gives there, with E = X - L1 - L2 + 1,
+//     f2 = f0 (E^2 - K) / (2 N),   K = 1 + 2 L1 L2,   N^2 = L1 L2 (l1-1)(l1+2)(l2-1)(l2+2),
+// and the l3 recursion Q(l3+1) f2(l3+1) = 4 (2 l3 + 1) f2(l3) - Q(l3) f2(l3-1), solved for the
+// odd degree between two even ones, gives f2(l3+1)^2 = f0(l3)^2 q(l3+1) (E + E')^2 / (16 N^2),
+// E' being E at l3 + 2.  (Both differences of squares are of integers; the recursion of f2 in l3
+// was 29 FP64 operations per two degrees for everything, this is 22.)
+//
+// q(l3) = k (2 l1 + 1 - k) Y with k = l3 - d, Y = (2d + k)(2d + k + 2 l1 + 1): the first factor is
+// the same for every l2 of a row, Y steps by exact integer differences.  The sums sum W'_l3 f^2
+// are accumulated in Horner form, G <- G q(l3) + W' R (...), and divided by P once at the end.
+// P grows by at most S^4 / 4 < 2^66 per two degrees (S = l1 + l2 + 1 < 2^17); every 8 pairs of
+// degrees all are rescaled by a power of two (exact), so nothing leaves the FP64 range.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -27,99 +27,98 @@
 namespace gm {
 
 struct CoupleRun {
-    double F2, F2p, F0;      // F2 at the current even degree, at the one before it, F0 at the even degree
-    double P;                // pi^2 at the current even degree
-    double G00, G02, GE, GO;  // Horner sums: 0-0, 0-2, 2-2 even J (scale P), 2-2 odd J (scale of the odd chain)
-    double A, B, st, c;      // A = (l3+1)^2 - d^2, B = S^2 - (l3+1)^2, st = 2 l3 + 3, c = 4 (2 l3 + 1)
-    double qe, qo, me;       // q at the current even degree, at the odd degree after it; P ratio of the last even step
+    double R, P;              // f0^2 = R / P at the current even degree
+    double G00, G02, GE, GO;  // Horner sums (scale P): 0-0, 0-2, 2-2 even J, 2-2 odd J, without 2 N, (2 N)^2, (4 N)^2
+    double Y, y1;             // Y at the next degree, its step
+    double E, sx, p2;         // E at the even degree, its step, E^2 - K
+    double me;                // P ratio of the last even step
+    double K, n2;             // n2 = 1 / N
 
     // g[p] = Gamma(p + 1/2) / (sqrt(pi) Gamma(p + 1)), p <= l2.
     __host__ __device__ void init(const double* __restrict__ g, int l1, int l2) {
         const int d = l2 - l1;
-        const double S2 = (double)(l1 + l2 + 1) * (double)(l1 + l2 + 1);
-        double w0 = sqrt(g[l1] * g[d] / ((2.0 * l2 + 1.0) * g[l2]));
-        if (l2 & 1) w0 = -w0;
-        double w2 = 0.0;
-        if (l1 >= 2)
-            w2 = w0 * sqrt((double)(l2 + 1) * (l2 + 2) * l1 * (l1 - 1) / ((double)l2 * (l2 - 1) * (l1 + 1) * (l1 + 2)));
-        F0 = w0;
-        F2 = w2;
-        F2p = 0.0;
+        const double a = l1, b = l2, n = 2.0 * a + 1.0, v = 2.0 * d + 1.0;
+        const double L1 = a * (a + 1.0), L2 = b * (b + 1.0);
+        R = g[l1] * g[d] / ((2.0 * b + 1.0) * g[l2]);
         P = 1.0;
         G00 = G02 = GE = GO = 0.0;
-        A = 2.0 * d + 1.0;
-        B = S2 - (double)(d + 1) * (d + 1);
-        st = 2.0 * d + 3.0;
-        c = 4.0 * (2.0 * d + 1.0);
-        qe = 0.0;
-        qo = 0.0;
+        Y = v * (v + n);
+        y1 = 2.0 * v + 1.0 + n;
+        E = (double)d * (d + 1.0) - L1 - L2 + 1.0;
+        sx = 4.0 * d + 6.0;
+        K = fma(2.0 * L1, L2, 1.0);
+        p2 = fma(E, E, -K);
         me = 1.0;
+        n2 = l1 >= 2 ? 1.0 / sqrt(L1 * L2 * ((a - 1.0) * (a + 2.0)) * ((b - 1.0) * (b + 2.0))) : 0.0;
     }
 
-    // Terms of the even degree l3 (weight we), step to l3 + 1, term of l3 + 1 (weight wo).
-    __host__ __device__ __forceinline__ void half_a(double we, double wo) {
-        const double t0 = we * F0, t2 = we * F2;
-        G00 = fma(G00, me, t0 * F0);
-        G02 = fma(G02, me, t0 * F2);
-        GE = fma(GE, me, t2 * F2);
-        qo = A * B;
-        A += st;
-        B -= st;
-        st += 2.0;
-        const double F2o = fma(c, F2, -(qe * F2p));
-        c += 8.0;
-        GO = fma(GO, qe * qo, (wo * F2o) * F2o);
-        F2p = F2o;
-    }
-
-    // Step from the odd degree to the next even one.
-    __host__ __device__ __forceinline__ void half_b() {
-        const double qn = A * B;
-        A += st;
-        B -= st;
-        st += 2.0;
-        const double F2n = fma(c, F2p, -(qo * F2));
-        c += 8.0;
-        F0 = -qo * F0;
-        me = qo * qn;
-        P *= me;
-        F2 = F2n;
-        qe = qn;
-    }
-
-    // Terms of the last (even) degree.
+    // Terms of an even degree.
     __host__ __device__ __forceinline__ void even_term(double we) {
-        const double t0 = we * F0, t2 = we * F2;
-        G00 = fma(G00, me, t0 * F0);
-        G02 = fma(G02, me, t0 * F2);
-        GE = fma(GE, me, t2 * F2);
+        const double t = we * R, t2 = t * p2;
+        G00 = fma(G00, me, t);
+        G02 = fma(G02, me, t2);
+        GE = fma(GE, me, t2 * p2);
     }
 
-    // Exact power-of-two rescale bringing P into [1/2, 2).
+    // Terms of the even degree l3 = d + k (weight we) and of l3 + 1 (weight wo);
+    // ko = (k + 1) (2 l1 - k).  Past the last degree (on false, zero weights) R stays.
+    __host__ __device__ __forceinline__ void half_a(double we, double wo, double ko, bool on = true) {
+        even_term(we);
+        R *= on ? ko * Y : 1.0;
+        Y += y1;
+        y1 += 2.0;
+        const double En = E + sx, h = E + En;
+        E = En;
+        sx += 8.0;
+        GO = fma(GO, me, (wo * R * h) * h);
+    }
+
+    // Step to the next even degree, ke = (k + 2) (2 l1 - 1 - k); past the last degree (on false)
+    // the sums keep their scale.
+    __host__ __device__ __forceinline__ void half_b(double ke, bool on = true) {
+        me = on ? ke * Y : 1.0;
+        Y += y1;
+        y1 += 2.0;
+        P *= me;
+        p2 = fma(E, E, -K);
+    }
+
+    // Exact power-of-two rescale bringing P into [1/2, 1).
     __host__ __device__ __forceinline__ void rescale() {
         int e;
         (void)frexp(P, &e);
-        const int h = e >> 1;
-        F2 = ldexp(F2, -h);
-        F2p = ldexp(F2p, -h);
-        F0 = ldexp(F0, -h);
-        P = ldexp(P, -2 * h);
-        G00 = ldexp(G00, -2 * h);
-        G02 = ldexp(G02, -2 * h);
-        GE = ldexp(GE, -2 * h);
-        GO = ldexp(GO, -2 * h);
+        R = ldexp(R, -e);
+        P = ldexp(P, -e);
+        G00 = ldexp(G00, -e);
+        G02 = ldexp(G02, -e);
+        GE = ldexp(GE, -e);
+        GO = ldexp(GO, -e);
     }
 
-    // Row sums (a00, a02, aE, aO).  ended_even: the last degree was even (then the odd chain
-    // ended one degree earlier, at pi^2 = P / qe); otherwise it ended at P * qo.
+    // Row sums (a00, a02, aE, aO).  ended_even: the last degree was even, so the odd sum is one
+    // even step behind.
     __host__ __device__ void finish(bool ended_even, double s[4]) const {
-        const double ri = 1.0 / P;
+        const double ri = 1.0 / P, h = 0.5 * n2;
         s[0] = G00 * ri;
-        s[1] = G02 * ri;
-        s[2] = GE * ri;
-        s[3] = ended_even ? GO * qe * ri : GO * ri / qo;
+        s[1] = G02 * ri * h;
+        s[2] = GE * ri * h * h;
+        s[3] = (ended_even ? GO * me : GO) * ri * (0.25 * h) * h;
     }
 };
+
+// The factor k (2 l1 + 1 - k) of q.
+__host__ __device__ __forceinline__ double couple_kappa(int k, int l1) { return (double)k * (double)(2 * l1 + 1 - k); }
+
+// A window that stages the factors k0 + 1 .. k0 + 64 with the weights returns them by kappa(t);
+// any other has them computed.
+template <class Win>
+__host__ __device__ __forceinline__ auto couple_kappa_at(const Win& w, int t, int, int) -> decltype(w.kappa(t)) {
+    return w.kappa(t);
+}
+template <class Win>
+__host__ __device__ __forceinline__ double couple_kappa_at(const Win&, int, long k, int l1) {
+    return couple_kappa((int)k, l1);
+}
 
 // Degrees l3 = d .. min(l1 + l2, lmax_w) of one pair, W' read from Wp; s = (a00, a02, aE, aO).
 __host__ __device__ inline void couple_pair(const double* __restrict__ Wp, int lmax_w, const double* __restrict__ g,
@@ -137,15 +136,15 @@ __host__ __device__ inline void couple_pair(const double* __restrict__ Wp, int l
     const int nfull = odd ? np : np - 1;
     int l3 = d;
     for (int j = 0; j < nfull; ++j) {
-        r.half_a(Wp[l3], Wp[l3 + 1]);
-        r.half_b();
+        r.half_a(Wp[l3], Wp[l3 + 1], couple_kappa(2 * j + 1, l1));
+        r.half_b(couple_kappa(2 * j + 2, l1));
         l3 += 2;
-        if ((j & 3) == 3) r.rescale();
+        if ((j & 7) == 7) r.rescale();
     }
     if (odd)
         r.even_term(Wp[l3]);
     else
-        r.half_a(Wp[l3], Wp[l3 + 1]);
+        r.half_a(Wp[l3], Wp[l3 + 1], couple_kappa(2 * nfull + 1, l1));
     r.finish(odd, s);
 }
 
@@ -170,8 +169,8 @@ __host__ __device__ inline void couple_decode(int64_t item, int L, int& l1, int&
 
 // One lane of a wave's item: row l1, columns l2 = l2_0 + lane (l2_0 >= l1).  All lanes run
 // the degree count of lane 0 (the smallest d, so the longest row): a lane with fewer
-// degrees in the window reads zeros past lmax_w (the window is zero-padded), and every lane
-// stays inside its triangle (l3 <= l1 + l2).  Win supplies W' per lane: stage(k0) loads
+// degrees in the window reads zeros past lmax_w (the window is zero-padded) and leaves its sums
+// unscaled from there, and every lane stays inside its triangle (l3 <= l1 + l2).  Win supplies W' per lane: stage(k0) loads
 // W'[d0 + k0 + t], t < 128, d0 = l2_0 - l1 (zero past lmax_w), and at(t) returns entry t;
 // lane i at degree l3 = d0 + i + k reads entry i + k - k0, with k0 = 64 floor(k / 64).
 // Lanes with l2 >= L run the row of l2 = L - 1; the caller stores only the lanes it owns.
@@ -192,28 +191,38 @@ __host__ __device__ inline void couple_wave_lane(Win& win, int lmax_w, const dou
     const int nfull = odd ? np : np - 1;
     win.stage(0);
     int p = 0;  // pair index: degrees d + 2p, d + 2p + 1
-    for (; p + 4 <= nfull; p += 4) {
+    auto kappa = [&](int q, int u) { return couple_kappa_at(win, 2 * (q & 31) + u - 1, 2 * q + u, l1); };
+    auto pair = [&](int q, int last) {  // last: pairs after which the lane has ended
+        const int o = lane + 2 * (q & 31);
+        r.half_a(win.at(o), win.at(o + 1), kappa(q, 1), q <= last);
+        r.half_b(kappa(q, 2), q < last);
+    };
+    // full pairs of this lane, and of the lane with the fewest (all equal unless the window ends)
+    const int nl = min(l1 + l2, lmax_w) - (l2 - l1) + 1, mine = nl > 0 ? (nl - 1) >> 1 : 0;
+    const int n63 = min(l1 + l2_0 + 63, lmax_w) - (d0 + 63) + 1;
+    const int all = min(n63 > 0 ? (n63 - 1) >> 1 : 0, nfull);
+    for (; p + 8 <= all; p += 8) {
         if (p && (p & 31) == 0) win.stage(2 * p);
-        const int o = lane + 2 * (p & 31);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            r.half_a(win.at(o + 2 * u), win.at(o + 2 * u + 1));
-            r.half_b();
-        }
+        for (int u = 0; u < 8; ++u) pair(p + u, p + 8);
+        r.rescale();
+    }
+    for (; p + 8 <= nfull; p += 8) {
+        if (p && (p & 31) == 0) win.stage(2 * p);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) pair(p + u, mine);
         r.rescale();
     }
     for (; p < nfull; ++p) {
         if (p && (p & 31) == 0) win.stage(2 * p);
-        const int o = lane + 2 * (p & 31);
-        r.half_a(win.at(o), win.at(o + 1));
-        r.half_b();
+        pair(p, mine);
     }
     if (p && (p & 31) == 0) win.stage(2 * p);
     const int o = lane + 2 * (p & 31);
     if (odd)
         r.even_term(win.at(o));
     else
-        r.half_a(win.at(o), win.at(o + 1));
+        r.half_a(win.at(o), win.at(o + 1), kappa(p, 1), p <= mine);
     r.finish(odd, s);
 }
 
