@@ -80,17 +80,26 @@ __global__ void k_bin_cell(const double* __restrict__ cl, int64_t ld, const int*
     out[(int64_t)c * nb + b] = s;
 }
 
-// out[b1][b2] = sum_{e1 in b1, e2 in b2} wout[e1] M[ells[e1]][ells[e2]] tin[e2].  Bound: latency of
-// the matrix's words (one row after the other before: 115 us for a 3072 x 3072 block, 4 degrees a
-// bin; kBinRows rows together: 64 us).
-constexpr int kBinRows = 4;
+// Binned coupling matrix: for each block M and its slots (c1, c2, sign),
+//   out[b1 ncls + c1][b2 ncls + c2] = sign sum_{e1 in b1, e2 in b2} wout[e1] M[ells[e1]][ells[e2]] tin[e2].
+// blockIdx.z = block of the list.  Bound: latency of the matrix's words (one row after the other
+// before: 115 us for a 3072 x 3072 block, 4 degrees a bin; kBinRows rows together: 64 us).  All
+// blocks and slots are one launch: eight slots of two blocks were 2 + 16 launches.
+constexpr int kBinRows = 4, kBinBlocks = 16, kBinSlots = 16;
 
-__global__ void k_bin_block(const double* __restrict__ M, int L, const int* __restrict__ ells,
-                            const int* __restrict__ bstart, int nb, const double* __restrict__ wout,
-                            const double* __restrict__ tin, double* __restrict__ out) {
+struct BinBlocks {
+    const double* M[kBinBlocks];
+    int nslots;
+    signed char block[kBinSlots], c1[kBinSlots], c2[kBinSlots], sign[kBinSlots];
+};
+
+__global__ void k_bin_blocks(BinBlocks bb, int L, const int* __restrict__ ells, const int* __restrict__ bstart, int nb,
+                             const double* __restrict__ wout, const double* __restrict__ tin, int ncls,
+                             double* __restrict__ out) {
     const int b2 = blockIdx.x * blockDim.x + threadIdx.x;
-    const int b1 = blockIdx.y;
+    const int b1 = blockIdx.y, z = blockIdx.z;
     if (b2 >= nb) return;
+    const double* __restrict__ M = bb.M[z];
     double s = 0.0;
     const int end = bstart[b1 + 1];
     for (int e1 = bstart[b1]; e1 < end; e1 += kBinRows) {
@@ -111,7 +120,10 @@ __global__ void k_bin_block(const double* __restrict__ M, int L, const int* __re
         for (int u = 0; u < kBinRows; ++u)
             if (e1 + u < end) s += wout[e1 + u] * r[u];
     }
-    out[(int64_t)b1 * nb + b2] = s;
+    for (int k = 0; k < bb.nslots; ++k)
+        if (bb.block[k] == z)
+            out[((int64_t)b1 * ncls + bb.c1[k]) * ((int64_t)nb * ncls) + (int64_t)b2 * ncls + bb.c2[k]] =
+                bb.sign[k] < 0 ? -s : s;
 }
 
 }  // namespace
@@ -206,13 +218,40 @@ extern "C" int gm_bin_cell(const double* cl, int64_t ncl, int64_t ld, const int3
     return check_launch("gm_bin_cell");
 }
 
+extern "C" int gm_bin_blocks(const double* const* blocks, int64_t nblocks, int64_t lmax, const int32_t* ells,
+                             const int32_t* band_start, int64_t nbands, const double* wout, const double* tin,
+                             int64_t ncls, const int32_t* slots, int64_t nslots, double* out, void* stream) {
+    if (!blocks || !ells || !band_start || !wout || !tin || !slots || !out)
+        return fail(GM_E_ARG, "gm_bin_blocks: null pointer");
+    if (lmax < 0 || nbands < 1 || ncls < 1 || ncls > 127) return fail(GM_E_ARG, "gm_bin_blocks: bad sizes");
+    if (nblocks < 1 || nblocks > kBinBlocks || nslots < 1 || nslots > kBinSlots)
+        return fail(GM_E_ARG, "gm_bin_blocks: at most %d blocks and %d slots", kBinBlocks, kBinSlots);
+    BinBlocks bb{};
+    bb.nslots = (int)nslots;
+    for (int64_t k = 0; k < nblocks; ++k) {
+        if (!blocks[k]) return fail(GM_E_ARG, "gm_bin_blocks: null pointer");
+        bb.M[k] = blocks[k];
+    }
+    for (int64_t k = 0; k < nslots; ++k) {
+        const int32_t* v = slots + 4 * k;
+        if (v[0] < 0 || v[0] >= nblocks || v[1] < 0 || v[1] >= ncls || v[2] < 0 || v[2] >= ncls || (v[3] != 1 && v[3] != -1))
+            return fail(GM_E_ARG, "gm_bin_blocks: bad slot %lld", (long long)k);
+        bb.block[k] = (signed char)v[0];
+        bb.c1[k] = (signed char)v[1];
+        bb.c2[k] = (signed char)v[2];
+        bb.sign[k] = (signed char)v[3];
+    }
+    hipLaunchKernelGGL(k_bin_blocks, dim3((unsigned)((nbands + 63) / 64), (unsigned)nbands, (unsigned)nblocks), dim3(64),
+                       0, (hipStream_t)stream, bb, (int)(lmax + 1), ells, band_start, (int)nbands, wout, tin, (int)ncls, out);
+    return check_launch("gm_bin_blocks");
+}
+
 extern "C" int gm_bin_block(const double* M, int64_t lmax, const int32_t* ells, const int32_t* band_start,
                             int64_t nbands, const double* wout, const double* tin, double* out, void* stream) {
     if (!M || !ells || !band_start || !wout || !tin || !out) return fail(GM_E_ARG, "gm_bin_block: null pointer");
     if (lmax < 0 || nbands < 1) return fail(GM_E_ARG, "gm_bin_block: bad sizes");
-    hipLaunchKernelGGL(k_bin_block, dim3((unsigned)((nbands + 63) / 64), (unsigned)nbands), dim3(64), 0,
-                       (hipStream_t)stream, M, (int)(lmax + 1), ells, band_start, (int)nbands, wout, tin, out);
-    return check_launch("gm_bin_block");
+    const int32_t slot[4] = {0, 0, 0, 1};
+    return gm_bin_blocks(&M, 1, lmax, ells, band_start, nbands, wout, tin, 1, slot, 1, out, stream);
 }
 
 // ------------------------------------------------------------------ content fingerprint

@@ -9,7 +9,7 @@ Restates ``gmaster/workspaces.py``:
 * the Toeplitz approximation (``:520-590, :1125-1194, :1834-1840``) -- kernels
   ``gm_coupling_pairs`` (exact entries only) and ``gm_toeplitz`` (the fill);
 * the slot / sign layout of the blocks (``:1851-1903``), binning with weights, f_ell and
-  beams (``:1452-1470, :292-310``) -- kernel ``gm_bin_block``;
+  beams (``:1452-1470, :292-310``) -- kernel ``gm_bin_blocks``;
 * ``decouple_cell`` (``:2106-2147``): binned spectra (``gm_bin_cell``) and an FP64 LU
   solve of the binned MCM: its LU factors (``gm_lu_factor``: blocked, without row
   exchanges, with a flag that falls back to ``torch.linalg.lu_factor`` when partial
@@ -17,6 +17,7 @@ Restates ``gmaster/workspaces.py``:
   ``decouple_cell`` (``gm_lu_solve``) and by the bandpower windows (getrs).
 """
 
+import ctypes
 import hashlib
 
 import numpy as np
@@ -598,15 +599,14 @@ class NmtWorkspace:
         tin = (beam[d["ells"].long()] * d["inv_f"]).contiguous()
         nb, ncls = self.nbands, self.ncls
         st = _lib.stream_ptr(dev)
-        binned = {}
-        for name in {b for b, _, _ in self.layout}:
-            out = torch.empty((nb, nb), dtype=torch.float64, device=dev)
-            _lib.call("gm_bin_block", _lib.ptr(self.blocks[name]), self.lmax, _lib.ptr(d["ells"]), _lib.ptr(d["start"]),
-                      nb, _lib.ptr(d["w"]), _lib.ptr(tin), _lib.ptr(out), st)
-            binned[name] = out
+        names = sorted({name for name, _, _ in self.layout})
+        ptrs = (ctypes.c_void_p * len(names))(*[_lib.ptr(self.blocks[name]) for name in names])
+        slots = (ctypes.c_int32 * (4 * len(self.layout)))(
+            *[v for name, (c1, c2), sign in self.layout for v in (names.index(name), c1, c2, int(sign))])
         mb = torch.zeros((nb, ncls, nb, ncls), dtype=torch.float64, device=dev)
-        for name, (c1, c2), sign in self.layout:
-            mb[:, c1, :, c2] += sign * binned[name]
+        _lib.call("gm_bin_blocks", ctypes.cast(ptrs, ctypes.c_void_p), len(names), self.lmax, _lib.ptr(d["ells"]),
+                  _lib.ptr(d["start"]), nb, _lib.ptr(d["w"]), _lib.ptr(tin), ncls, ctypes.cast(slots, ctypes.c_void_p),
+                  len(self.layout), _lib.ptr(mb), st)
         mb = mb.reshape(nb * ncls, nb * ncls)
         if self.norm_type:
             mb = self.wawb * torch.eye(nb * ncls, dtype=torch.float64, device=dev)

@@ -307,6 +307,13 @@ int gm_lu_solve(const double* LU, const double* LUT, int64_t n, double* B, int64
 int gm_bin_block(const double* M, int64_t lmax, const int32_t* ells, const int32_t* band_start,
                  int64_t nbands, const double* wout, const double* tin, double* out, void* stream);
 
+/* The same for every block of a binned coupling matrix, into its slots: slots holds (block, c1,
+ * c2, sign) per slot, out[b1 ncls + c1][b2 ncls + c2] = sign x binned block (rows of nbands ncls).
+ * blocks (device pointers) and slots are host arrays, at most 16 of each; other slots are left. */
+int gm_bin_blocks(const double* const* blocks, int64_t nblocks, int64_t lmax, const int32_t* ells,
+                  const int32_t* band_start, int64_t nbands, const double* wout, const double* tin,
+                  int64_t ncls, const int32_t* slots, int64_t nslots, double* out, void* stream);
+
 /* Binned spectra: out[c][b] = sum_{l in b} w[l] cl[c][l].  Replaces gmaster/bins.py:15-20. */
 int gm_bin_cell(const double* cl, int64_t ncl, int64_t ld, const int32_t* ells,
                 const int32_t* band_start, int64_t nbands, const double* w, double* out, void* stream);

@@ -56,3 +56,37 @@ def test_bin_block_edges(nlb):
         sel[i, start[i]:start[i + 1]] = 1.0
     ref = sel @ t @ sel.T
     assert float((out - ref).abs().max()) <= (nlb * nlb + 4) * 2 * EPS * float(t.abs().max())
+
+
+@pytest.mark.parametrize("ncls,nslots", [(1, 1), (4, 8), (7, 11)])
+def test_bin_blocks_fill_their_slots(ncls, nslots):
+    """gm_bin_blocks against gm_bin_block block by block: every slot, its sign, and nothing else."""
+    import ctypes
+
+    from gmaster_amd import _lib
+
+    L, nlb = 70, 3
+    st = _lib.stream_ptr("cuda")
+    g = torch.Generator("cuda").manual_seed(ncls)
+    nblk = min(9, nslots)
+    Ms = [torch.randn((L, L), dtype=torch.float64, device="cuda", generator=g) for _ in range(nblk)]
+    start = list(range(0, L - 1, nlb)) + [L - 1]
+    ells = torch.arange(1, L, dtype=torch.int32, device="cuda")
+    bs = torch.tensor(start, dtype=torch.int32, device="cuda")
+    wo, ti = (torch.rand(L - 1, dtype=torch.float64, device="cuda", generator=g) for _ in range(2))
+    nb = len(start) - 1
+    at = [(k // ncls, (3 * k) % ncls) if ncls > 1 else (0, 0) for k in range(nslots)]
+    assert len(set(at)) == nslots
+    slots = [(k % nblk, c1, c2, -1 if k % 3 == 2 else 1) for k, (c1, c2) in enumerate(at)]
+    ref = torch.full((nb, ncls, nb, ncls), 5.0, dtype=torch.float64, device="cuda")
+    out = ref.clone()
+    one = torch.empty((nb, nb), dtype=torch.float64, device="cuda")
+    for k, c1, c2, sign in slots:
+        _lib.call("gm_bin_block", _lib.ptr(Ms[k]), L - 1, _lib.ptr(ells), _lib.ptr(bs), nb, _lib.ptr(wo), _lib.ptr(ti),
+                  _lib.ptr(one), st)
+        ref[:, c1, :, c2] = sign * one
+    ptrs = (ctypes.c_void_p * nblk)(*[m.data_ptr() for m in Ms])
+    flat = (ctypes.c_int32 * (4 * nslots))(*[v for s in slots for v in s])
+    _lib.call("gm_bin_blocks", ctypes.cast(ptrs, ctypes.c_void_p), nblk, L - 1, _lib.ptr(ells), _lib.ptr(bs), nb,
+              _lib.ptr(wo), _lib.ptr(ti), ncls, ctypes.cast(flat, ctypes.c_void_p), nslots, _lib.ptr(out), st)
+    assert torch.equal(out, ref)
