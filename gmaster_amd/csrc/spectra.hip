@@ -271,14 +271,29 @@ __global__ void k_fingerprint_clear(unsigned long long* out) {
 
 // Two order-independent 64-bit sums of position-keyed word hashes; any change of one word
 // changes both sums unless two independent 64-bit hashes collide.
-__global__ void k_fingerprint(const uint64_t* __restrict__ w, int64_t nwords, const unsigned char* __restrict__ tail,
+// Bound: HBM and the hashes' multiplications for large buffers.  The sums meet in two words, so
+// a workgroup adds once, and at most kFingerBlocks workgroups run: one atomic per wave of 2048
+// workgroups queued up on them for 200 us at any size above 4 MiB (Nside 64, 384 KiB: 21 -> 4;
+// Nside 1024, 96 MiB: 208 -> 33).
+constexpr int kFingerThreads = 1024, kFingerBlocks = 256;
+
+__global__ __launch_bounds__(kFingerThreads) void k_fingerprint(const uint64_t* __restrict__ w, int64_t nwords, const unsigned char* __restrict__ tail,
                               int ntail, unsigned long long* out) {
     uint64_t s1 = 0, s2 = 0;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nwords; i += stride) {
-        const uint64_t h = mix64(w[i] ^ mix64((uint64_t)i + 0x9e3779b97f4a7c15ull));
-        s1 += h;
-        s2 += mix64(h ^ 0x632be59bd9b4e019ull);
+    for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < nwords; i0 += 4 * stride) {
+        uint64_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = w[i0 + u * stride < nwords ? i0 + u * stride : i0];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t i = i0 + u * stride;
+            if (i < nwords) {
+                const uint64_t h = mix64(v[u] ^ mix64((uint64_t)i + 0x9e3779b97f4a7c15ull));
+                s1 += h;
+                s2 += mix64(h ^ 0x632be59bd9b4e019ull);
+            }
+        }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && ntail > 0) {
         uint64_t t = 0;
@@ -291,9 +306,16 @@ __global__ void k_fingerprint(const uint64_t* __restrict__ w, int64_t nwords, co
         s1 += __shfl_down(s1, off);
         s2 += __shfl_down(s2, off);
     }
+    __shared__ uint64_t part[2][kFingerThreads / 64];
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&out[0], (unsigned long long)s1);
-        atomicAdd(&out[1], (unsigned long long)s2);
+        part[0][threadIdx.x >> 6] = s1;
+        part[1][threadIdx.x >> 6] = s2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        uint64_t t = 0;
+        for (int k = 0; k < kFingerThreads / 64; ++k) t += part[threadIdx.x][k];
+        atomicAdd(&out[threadIdx.x], (unsigned long long)t);
     }
 }
 
@@ -309,10 +331,10 @@ extern "C" int gm_fingerprint(const void* data, int64_t nbytes, uint64_t* out, v
     hipLaunchKernelGGL(k_fingerprint_clear, dim3(1), dim3(64), 0, st, o);
     const int64_t nwords = nbytes / 8;
     const int ntail = (int)(nbytes - nwords * 8);
-    int64_t blocks = (nwords + 255) / 256;
-    if (blocks > 2048) blocks = 2048;
+    int64_t blocks = (nwords + kFingerThreads - 1) / kFingerThreads;
+    if (blocks > kFingerBlocks) blocks = kFingerBlocks;
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_fingerprint, dim3((unsigned)blocks), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_fingerprint, dim3((unsigned)blocks), dim3(kFingerThreads), 0, st,
                        reinterpret_cast<const uint64_t*>(data), nwords,
                        reinterpret_cast<const unsigned char*>(data) + nwords * 8, ntail, o);
     return check_launch("gm_fingerprint");
