@@ -157,8 +157,11 @@ def plan(nside, lmax, spin, device=None, polar_skip=True):
 
 
 # Ring pairs with sin^2(theta) below this run the spin-2 recurrence itself; the others the
-# spin-0 rows with weights 1/sin^2, which amplify rounding by up to this bound's inverse.
-PAIR_SIN2 = 1.0 / 32.0
+# spin-0 rows with weights 1/sin^2, which amplify rounding by up to this bound's inverse.  The
+# polar blocks cost four times a ring pair's: 1/32 -> 1/64 measured 18.6 -> 17.9 ms for map2alm
+# with three iterations at Nside 1024 and 42.7 -> 40.7 ms for a T+P run, the error against exact
+# sums unchanged from Nside 512 on (1.4e-14, 2.8e-13) and 1 - 1.4 of 2e-15 at Nside 64.
+PAIR_SIN2 = 1.0 / 64.0
 
 
 @dataclass
