@@ -34,7 +34,7 @@
 // Synthesis (k_bat_syn): as the spin-0 mixed synthesis, one v_mfma_f32_4x4x1f32 per
 // (degree, ring set, 4 channels), lanes = ring pairs, E/O accumulators; the epilogue
 // divides the spin-2 sums by s^2 and writes F+(+-m) = Q + iU, conj(Q) + i conj(U).  Polar
-// ring pairs use an FP64 vector-ALU variant (k_bat_syn64).  Tables run to degree lmax + 2
+// ring pairs use an FP64 vector-ALU variant (bat_syn64).  Tables run to degree lmax + 2
 // (the folded plain part reaches one degree past lmax + 1).
 #include "common.h"
 #include "recurrence.h"
@@ -692,22 +692,28 @@ __global__ __launch_bounds__(256) void k_bat_prep(const double2* __restrict__ al
 
 __device__ inline f4 mfma4(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0); }
 
-// Writes of ring pair j's outputs: spin-0 channel values (N = E + O, S = E - O) and the
-// spin-2 components Q, U (1/s^2 part + plain part) as F+(m) = Q + iU, F+(-m) = conj Q + i conj U.
-__device__ inline void put_spin2(double2* __restrict__ spec2, int64_t ld2, int L, int m, int ring, double qr, double qi,
-                                 double ur, double ui) {
+// F+(m) = Q + iU and F+(-m) = conj Q + i conj U of one ring, from the sums (Q re, Q im, U re, U im)
+// times rs.  The fused operations are spelled out: the batched residuals' operand splits see the
+// last bit of a spectrum, and the compiler's choice of which product to fuse is not stable.
+__device__ inline void put_spin2(double2* __restrict__ spec2, int64_t ld2, int L, int m, int ring, const double (&s)[4],
+                                 double rs) {
+#pragma clang fp contract(off)
     double2* row = spec2 + (int64_t)ring * ld2 + (L - 1);
-    row[m] = make_double2(qr - ui, qi + ur);
+    const double qr = s[0] * rs, qi = s[1] * rs, ur = s[2] * rs, ui = s[3] * rs;
+    row[m] = make_double2(fma(s[0], rs, -ui), fma(s[1], rs, ur));
     if (m) row[-m] = make_double2(qr + ui, ur - qi);
 }
 
+// One workgroup of FP32 synthesis: ring pairs jbeg + blk CH .. + CH - 1 of order m.  cst: LDS of
+// syn_words32 floats per wave.
+template <int K0, int K2> constexpr int syn_words32() { return Chan<K0, K2>::syn_stride * (kTile + 4); }
+
 template <int K0, int K2, int NW, int R>
-__global__ __launch_bounds__(64 * NW, GM_BAT_SYN_WAVES) void k_bat_syn(const double* __restrict__ coef, int nside, int L,
-                                                     const double* __restrict__ alpha, const double* __restrict__ smant,
-                                                     const int* __restrict__ sexp, const int* __restrict__ nact,
-                                                     int jbeg, int jend, double2* __restrict__ spec0, int64_t ld0,
-                                                     int64_t smap0, double2* __restrict__ spec2, int64_t ld2,
-                                                     int64_t smap2) {
+__device__ __forceinline__ void bat_syn32(const double* __restrict__ coef, int nside, int L,
+                                          const double* __restrict__ alpha, const double* __restrict__ smant,
+                                          const int* __restrict__ sexp, const int* __restrict__ nact, int m, int blk,
+                                          int jbeg, int jend, double2* __restrict__ spec0, int64_t ld0, int64_t smap0,
+                                          double2* __restrict__ spec2, int64_t ld2, int64_t smap2, float* cst) {
     typedef Chan<K0, K2> C;
     constexpr int NS = C::syn_stride;
     constexpr int NG = NS / 4;
@@ -716,12 +722,10 @@ __global__ __launch_bounds__(64 * NW, GM_BAT_SYN_WAVES) void k_bat_syn(const dou
     constexpr int NV = kTile * NS / 64;  // coefficients each lane stages per block
     constexpr int SR = kTile + 4;        // staged row: one channel, kTile degrees (+ padding)
     static_assert(kTile * NS % 64 == 0, "a block of coefficients must split evenly over a wave");
-    // per wave: the FP32 coefficients of kTile degrees, [channel][degree]
-    __shared__ __align__(16) float cst[NW][NS * SR];
+    static_assert(NS * SR == syn_words32<K0, K2>(), "LDS words");
     const int Lt = L + kTabExtra;
-    const int m = blockIdx.y;
     const int jhi = min(nact[m], jend);
-    const int j0 = jbeg + blockIdx.x * CH;
+    const int j0 = jbeg + blk * CH;
     const int w = threadIdx.x >> 6, ln = threadIdx.x & 63;
     const int q4 = threadIdx.x & 3, qbase = threadIdx.x & ~3;
 
@@ -755,7 +759,7 @@ __global__ __launch_bounds__(64 * NW, GM_BAT_SYN_WAVES) void k_bat_syn(const dou
         // when staged, and alpha past L keeps mu finite for the discarded degrees
         const double* al = alpha + table_base(m, Lt) - m;
         const double* cf = coef + (table_base(m, Lt) - m) * NS;
-        float* my = cst[w];
+        float* my = cst + w * (NS * SR);  // the FP32 coefficients of kTile degrees, [channel][degree]
         double pf[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) pf[v] = cf[(int64_t)m * NS + v * 64 + ln];
@@ -867,23 +871,22 @@ __global__ __launch_bounds__(64 * NW, GM_BAT_SYN_WAVES) void k_bat_syn(const dou
 // registers (no cross-lane exchange in the epilogue).  The coefficients of each block of
 // kTile degrees are staged in a wave-private LDS buffer (one coalesced load, the next
 // block's issued half a block ahead) and read back as broadcasts.
+template <int K0, int K2> constexpr int syn_words64() { return kTile * Chan<K0, K2>::syn_stride; }
+
 template <int K0, int K2, int NW, int R>
-__global__ __launch_bounds__(64 * NW) void k_bat_syn64(const double* __restrict__ coef, int nside, int L,
-                                                       const double* __restrict__ alpha,
-                                                       const double* __restrict__ smant, const int* __restrict__ sexp,
-                                                       const int* __restrict__ nact, int jbeg, int jend,
-                                                       double2* __restrict__ spec0, int64_t ld0, int64_t smap0,
-                                                       double2* __restrict__ spec2, int64_t ld2, int64_t smap2) {
+__device__ __forceinline__ void bat_syn64(const double* __restrict__ coef, int nside, int L,
+                                          const double* __restrict__ alpha, const double* __restrict__ smant,
+                                          const int* __restrict__ sexp, const int* __restrict__ nact, int m, int blk,
+                                          int jbeg, int jend, double2* __restrict__ spec0, int64_t ld0, int64_t smap0,
+                                          double2* __restrict__ spec2, int64_t ld2, int64_t smap2, double* cst) {
     typedef Chan<K0, K2> C;
     constexpr int NS = C::syn_stride;
     constexpr int T = 64 * NW;
     constexpr int NV = kTile * NS / 64;  // coefficients each lane stages per block
     static_assert(kTile * NS % 64 == 0 && NS % 2 == 0, "blocks must split evenly over a wave");
-    __shared__ __align__(16) double cst[NW][kTile * NS];
     const int Lt = L + kTabExtra;
-    const int m = blockIdx.y;
     const int jhi = min(nact[m], jend);
-    const int j0 = jbeg + blockIdx.x * T * R;
+    const int j0 = jbeg + blk * T * R;
     double x[R], mu0[R], mu1[R];
     int kx[R];
     double acc[R][2][NS];
@@ -909,7 +912,7 @@ __global__ __launch_bounds__(64 * NW) void k_bat_syn64(const double* __restrict_
         anyinact = __any(anyinact);
         const double* al = alpha + table_base(m, Lt) - m;
         const double* cf = coef + (table_base(m, Lt) - m) * NS;
-        double* my = cst[threadIdx.x >> 6];
+        double* my = cst + (threadIdx.x >> 6) * (kTile * NS);
         const int ln = threadIdx.x & 63;
         double pf[NV];
 #pragma unroll
@@ -969,23 +972,41 @@ __global__ __launch_bounds__(64 * NW) void k_bat_syn64(const double* __restrict_
 #pragma unroll
         for (int f = 0; f < K2; ++f) {
             const int b = C::syn_base2 + 4 * f;
-            double nq[4], sq[4];
+            double n[4], u[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                nq[c] = (acc[t][0][b + c] + acc[t][1][b + c]) * rs;
-                sq[c] = (acc[t][0][b + c] - acc[t][1][b + c]) * rs;
+                n[c] = acc[t][0][b + c] + acc[t][1][b + c];
+                u[c] = acc[t][0][b + c] - acc[t][1][b + c];
             }
-            put_spin2(spec2 + f * smap2, ld2, L, m, r, nq[0], nq[1], nq[2], nq[3]);
-            if (j > 0) put_spin2(spec2 + f * smap2, ld2, L, m, rp, sq[0], sq[1], sq[2], sq[3]);
+            put_spin2(spec2 + f * smap2, ld2, L, m, r, n, rs);
+            if (j > 0) put_spin2(spec2 + f * smap2, ld2, L, m, rp, u, rs);
         }
     }
+}
+
+// Order blockIdx.y: workgroups 0 .. nb64 - 1 are polar ring pairs in FP64, the others FP32.
+template <int K0, int K2, int NW, int R, bool POL, bool MAIN>
+__global__ __launch_bounds__(64 * NW, MAIN ? GM_BAT_SYN_WAVES : 1) void k_bat_syn(
+    const double* __restrict__ coef, int nside, int L, const double* __restrict__ alpha, const double* __restrict__ smant,
+    const int* __restrict__ sexp, const int* __restrict__ nact, int jsplit, int nb64, double2* __restrict__ spec0,
+    int64_t ld0, int64_t smap0, double2* __restrict__ spec2, int64_t ld2, int64_t smap2) {
+    constexpr int W32 = MAIN ? syn_words32<K0, K2>() : 0, W64 = POL ? syn_words64<K0, K2>() : 0;
+    __shared__ __align__(16) double cst[NW * (W64 > W32 / 2 ? W64 : W32 / 2)];
+    const int m = blockIdx.y, b = blockIdx.x;
+    if (POL && (!MAIN || b < nb64))
+        bat_syn64<K0, K2, NW, 1>(coef, nside, L, alpha, smant, sexp, nact, m, b, jsplit, 2 * nside, spec0, ld0, smap0,
+                                 spec2, ld2, smap2, cst);
+    else
+        bat_syn32<K0, K2, NW, R>(coef, nside, L, alpha, smant, sexp, nact, m, POL ? b - nb64 : b, 0, jsplit, spec0, ld0,
+                                 smap0, spec2, ld2, smap2, reinterpret_cast<float*>(cst));
 }
 
 // ------------------------------------------------------------------ launch configuration
 constexpr int kAnaNW = GM_BAT_ANA_NW, kAnaR = GM_BAT_ANA_R;  // FP32 analysis: 512 ring pairs per workgroup
 constexpr int kAna64NW = 4;             // FP64 analysis: 256 ring pairs per workgroup
 constexpr int kSynNW = GM_BAT_SYN_NW, kSynR = GM_BAT_SYN_R;  // FP32 synthesis: 512 ring pairs per workgroup
-constexpr int kSyn64NW = 2, kSyn64R = 1;  // FP64 synthesis: 128 ring pairs per workgroup
+
+constexpr int kSyn64NW = 2;             // FP64 synthesis in a launch of its own: 128 ring pairs per workgroup
 
 constexpr int kAnaCH32 = 64 * kAnaNW * kAnaR, kAnaCH64 = 64 * kAna64NW;
 
@@ -1144,17 +1165,30 @@ extern "C" int gm_bat_syn(const double* coef, int64_t k0, int64_t k2, int64_t ns
     hipStream_t st = (hipStream_t)stream;
     auto* s0 = reinterpret_cast<double2*>(spec0);
     auto* s2 = reinterpret_cast<double2*>(spec2);
-    constexpr int CH = 64 * kSynNW * kSynR, CH64 = 64 * kSyn64NW * kSyn64R;
-    const int nb32 = (int)((jsplit + CH - 1) / CH), nb64 = (int)((2 * nside - jsplit + CH64 - 1) / CH64);
+    // The polar pairs are a few long FP64 recurrences: in a launch of their own they leave the chip
+    // empty, so up to Nside 1024 both share one (2 polarisation fields at Nside 128: 80 -> 57 us,
+    // 512: 600 -> 544; 2 maps and a field at 1024: 3.27 -> 3.18 ms).  Their registers cost the FP32
+    // workgroups a wave per SIMD, which is more at Nside 2048 (18.0 -> 19.0 ms); eight maps do not
+    // fit the shared kernel's registers (512: 1.0 -> 3.8 ms).
+    constexpr int CH = 64 * kSynNW * kSynR;
+    const int np = (int)(2 * nside - jsplit), nb32 = (int)((jsplit + CH - 1) / CH);
+#define GM_SYN(NW, POL, MAIN, B32)                                                                                      \
+    do {                                                                                                               \
+        const int nb64 = POL ? (np + 64 * (NW) - 1) / (64 * (NW)) : 0, blocks = nb64 + (B32);                           \
+        if (blocks > 0)                                                                                                \
+            hipLaunchKernelGGL((k_bat_syn<K0, K2, NW, kSynR, POL, MAIN>), dim3(blocks, (unsigned)L), dim3(64 * (NW)), 0, \
+                               st, coef, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, (int)jsplit, nb64,  \
+                               s0, ld0, smap0, s2, ld2, smap2);                                                        \
+    } while (0)
     GM_BAT_DISPATCH(K0, K2, {
-        if (nb32 > 0)
-            hipLaunchKernelGGL((k_bat_syn<K0, K2, kSynNW, kSynR>), dim3(nb32, (unsigned)L), dim3(64 * kSynNW), 0, st,
-                               coef, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, 0, (int)jsplit, s0, ld0,
-                               smap0, s2, ld2, smap2);
-        if (nb64 > 0)
-            hipLaunchKernelGGL((k_bat_syn64<K0, K2, kSyn64NW, kSyn64R>), dim3(nb64, (unsigned)L), dim3(64 * kSyn64NW), 0, st,
-                               coef, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, (int)jsplit,
-                               (int)(2 * nside), s0, ld0, smap0, s2, ld2, smap2);
+        constexpr bool fits = (Chan<K0, K2>::syn_stride <= 8);
+        if (fits && nside <= 1024) {
+            if constexpr (fits) GM_SYN(kSynNW, true, true, nb32);
+        } else {
+            GM_SYN(kSynNW, false, true, nb32);
+            GM_SYN(kSyn64NW, true, false, 0);
+        }
     })
+#undef GM_SYN
     return check_launch(name);
 }
