@@ -82,10 +82,15 @@ __global__ void k_bin_cell(const double* __restrict__ cl, int64_t ld, const int*
 
 // Binned coupling matrix: for each block M and its slots (c1, c2, sign),
 //   out[b1 ncls + c1][b2 ncls + c2] = sign sum_{e1 in b1, e2 in b2} wout[e1] M[ells[e1]][ells[e2]] tin[e2].
-// blockIdx.z = block of the list.  Bound: latency of the matrix's words (one row after the other
-// before: 115 us for a 3072 x 3072 block, 4 degrees a bin; kBinRows rows together: 64 us).  All
-// blocks and slots are one launch: eight slots of two blocks were 2 + 16 launches.
-constexpr int kBinRows = 4, kBinBlocks = 16, kBinSlots = 16;
+// blockIdx.z = block of the list, blockIdx.x = nbw bins b2.  One thread per column: its sum over
+// the rows of b1 (eight rows in flight), then the columns' products meet in LDS and one thread
+// per bin adds its own, 256 columns at a time.  Bound: HBM for wide matrices, else latency.  One
+// thread per bin read a cache line per column (16 degrees a bin: ten times the matrix's bytes,
+// 2.7 ms a block at lmax 12287 -> 0.21) and one row after the other (115 us for a
+// 3072 x 3072 block, 4 degrees a bin -> 19 us).  All blocks and slots are one launch: eight slots
+// of two blocks were 2 + 16 launches.
+constexpr int kBinBlocks = 16, kBinSlots = 16;
+template <int N> struct Rows { static constexpr int value = N; };
 
 struct BinBlocks {
     const double* M[kBinBlocks];
@@ -93,33 +98,47 @@ struct BinBlocks {
     signed char block[kBinSlots], c1[kBinSlots], c2[kBinSlots], sign[kBinSlots];
 };
 
-__global__ void k_bin_blocks(BinBlocks bb, int L, const int* __restrict__ ells, const int* __restrict__ bstart, int nb,
-                             const double* __restrict__ wout, const double* __restrict__ tin, int ncls,
-                             double* __restrict__ out) {
-    const int b2 = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_bin_blocks(BinBlocks bb, int L, const int* __restrict__ ells,
+                                                    const int* __restrict__ bstart, int nb,
+                                                    const double* __restrict__ wout, const double* __restrict__ tin,
+                                                    int ncls, int nbw, double* __restrict__ out) {
+    __shared__ double val[256];
+    const int tid = threadIdx.x;
     const int b1 = blockIdx.y, z = blockIdx.z;
-    if (b2 >= nb) return;
+    const int first = blockIdx.x * nbw, b2 = first + tid;
+    const bool mine = tid < nbw && b2 < nb;
     const double* __restrict__ M = bb.M[z];
+    const int lo = mine ? bstart[b2] : 0, hi = mine ? bstart[b2 + 1] : 0;
+    const int c_end = bstart[min(first + nbw, nb)];
+    const int r0 = bstart[b1], end = bstart[b1 + 1];
     double s = 0.0;
-    const int end = bstart[b1 + 1];
-    for (int e1 = bstart[b1]; e1 < end; e1 += kBinRows) {
-        const double* row[kBinRows];
-        double r[kBinRows];
-#pragma unroll
-        for (int u = 0; u < kBinRows; ++u) {
-            row[u] = M + (int64_t)ells[min(e1 + u, end - 1)] * L;
-            r[u] = 0.0;
-        }
-        for (int e2 = bstart[b2]; e2 < bstart[b2 + 1]; ++e2) {
+    for (int c0 = bstart[first]; c0 < c_end; c0 += 256) {
+        const int e2 = c0 + tid;
+        double v = 0.0;
+        if (e2 < c_end) {
             const int c = ells[e2];
-            const double t = tin[e2];
+            auto rows = [&](auto n, int e1) {
+                double m[n.value];
 #pragma unroll
-            for (int u = 0; u < kBinRows; ++u) r[u] += row[u][c] * t;
+                for (int u = 0; u < n.value; ++u) m[u] = M[(int64_t)ells[e1 + u] * L + c];
+#pragma unroll
+                for (int u = 0; u < n.value; ++u) v = fma(wout[e1 + u], m[u], v);
+            };
+            int e1 = r0;
+            for (; e1 + 8 <= end; e1 += 8) rows(Rows<8>{}, e1);
+            if (e1 + 4 <= end) {
+                rows(Rows<4>{}, e1);
+                e1 += 4;
+            }
+            for (; e1 < end; ++e1) rows(Rows<1>{}, e1);
+            v *= tin[e2];
         }
-#pragma unroll
-        for (int u = 0; u < kBinRows; ++u)
-            if (e1 + u < end) s += wout[e1 + u] * r[u];
+        val[tid] = v;
+        __syncthreads();
+        for (int e = max(lo, c0); e < min(hi, c0 + 256); ++e) s += val[e - c0];
+        __syncthreads();
     }
+    if (!mine) return;
     for (int k = 0; k < bb.nslots; ++k)
         if (bb.block[k] == z)
             out[((int64_t)b1 * ncls + bb.c1[k]) * ((int64_t)nb * ncls) + (int64_t)b2 * ncls + bb.c2[k]] =
@@ -241,8 +260,11 @@ extern "C" int gm_bin_blocks(const double* const* blocks, int64_t nblocks, int64
         bb.c2[k] = (signed char)v[2];
         bb.sign[k] = (signed char)v[3];
     }
-    hipLaunchKernelGGL(k_bin_blocks, dim3((unsigned)((nbands + 63) / 64), (unsigned)nbands, (unsigned)nblocks), dim3(64),
-                       0, (hipStream_t)stream, bb, (int)(lmax + 1), ells, band_start, (int)nbands, wout, tin, (int)ncls, out);
+    // 256 columns a workgroup: 64 bins of four degrees or more, 256 narrower ones (lmax 3071, bins of
+    // one degree: 128 us in 64s, 46 in 256s)
+    const int nbw = 3 * nbands > lmax + 1 ? 256 : 64;
+    hipLaunchKernelGGL(k_bin_blocks, dim3((unsigned)((nbands + nbw - 1) / nbw), (unsigned)nbands, (unsigned)nblocks), dim3(256),
+                       0, (hipStream_t)stream, bb, (int)(lmax + 1), ells, band_start, (int)nbands, wout, tin, (int)ncls, nbw, out);
     return check_launch("gm_bin_blocks");
 }
 
