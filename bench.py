@@ -630,7 +630,7 @@ def main():
             "gm_ring_fold_residual_c", "k_fold_s (Q + iU)", 3 * nring * (2 * L - 1) * 16,
             "synthesis + residual read, residual written")
     stage_roofs["coupling_fp64"] = flop_entry(
-        "gm_coupling", "k_coupling (exact 0-0, 0-2, 2-2 3j rows, plain FP64 form)", 24.0 * _n3j(lmax), PEAK_FP64,
+        "gm_coupling", "k_coupling (exact 0-0, 0-2, 2-2 3j rows, plain FP64 form)", 13.5 * _n3j(lmax), PEAK_FP64,
         "fp64 valu", stages_fp64)
     roofline_fp64 = roof(stages_fp64, False)
     ana0_ms = stages_fp64.get("gm_lat_ana_s0", {}).get("mean_ms", float("nan"))
