@@ -89,11 +89,11 @@ __global__ void k_bin_cell(const double* __restrict__ cl, int64_t ld, const int*
 // 2.7 ms a block at lmax 12287 -> 0.21) and one row after the other (115 us for a
 // 3072 x 3072 block, 4 degrees a bin -> 19 us).  All blocks and slots are one launch: eight slots
 // of two blocks were 2 + 16 launches.
-constexpr int kBinBlocks = 16, kBinSlots = 16;
+constexpr int kBinSlots = 16;  // of one launch
 template <int N> struct Rows { static constexpr int value = N; };
 
 struct BinBlocks {
-    const double* M[kBinBlocks];
+    const double* M[kBinSlots];
     int nslots;
     signed char block[kBinSlots], c1[kBinSlots], c2[kBinSlots], sign[kBinSlots];
 };
@@ -243,28 +243,37 @@ extern "C" int gm_bin_blocks(const double* const* blocks, int64_t nblocks, int64
     if (!blocks || !ells || !band_start || !wout || !tin || !slots || !out)
         return fail(GM_E_ARG, "gm_bin_blocks: null pointer");
     if (lmax < 0 || nbands < 1 || ncls < 1 || ncls > 127) return fail(GM_E_ARG, "gm_bin_blocks: bad sizes");
-    if (nblocks < 1 || nblocks > kBinBlocks || nslots < 1 || nslots > kBinSlots)
-        return fail(GM_E_ARG, "gm_bin_blocks: at most %d blocks and %d slots", kBinBlocks, kBinSlots);
-    BinBlocks bb{};
-    bb.nslots = (int)nslots;
-    for (int64_t k = 0; k < nblocks; ++k) {
+    if (nblocks < 1 || nslots < 1) return fail(GM_E_ARG, "gm_bin_blocks: bad sizes");
+    for (int64_t k = 0; k < nblocks; ++k)
         if (!blocks[k]) return fail(GM_E_ARG, "gm_bin_blocks: null pointer");
-        bb.M[k] = blocks[k];
-    }
     for (int64_t k = 0; k < nslots; ++k) {
         const int32_t* v = slots + 4 * k;
         if (v[0] < 0 || v[0] >= nblocks || v[1] < 0 || v[1] >= ncls || v[2] < 0 || v[2] >= ncls || (v[3] != 1 && v[3] != -1))
             return fail(GM_E_ARG, "gm_bin_blocks: bad slot %lld", (long long)k);
-        bb.block[k] = (signed char)v[0];
-        bb.c1[k] = (signed char)v[1];
-        bb.c2[k] = (signed char)v[2];
-        bb.sign[k] = (signed char)v[3];
     }
     // 256 columns a workgroup: 64 bins of four degrees or more, 256 narrower ones (lmax 3071, bins of
     // one degree: 128 us in 64s, 46 in 256s)
     const int nbw = 3 * nbands > lmax + 1 ? 256 : 64;
-    hipLaunchKernelGGL(k_bin_blocks, dim3((unsigned)((nbands + nbw - 1) / nbw), (unsigned)nbands, (unsigned)nblocks), dim3(256),
-                       0, (hipStream_t)stream, bb, (int)(lmax + 1), ells, band_start, (int)nbands, wout, tin, (int)ncls, nbw, out);
+    // kBinSlots slots a launch: every layout of the workspaces but one block per channel pair of a
+    // joint TEB workspace (49) is one launch
+    for (int64_t k0 = 0; k0 < nslots; k0 += kBinSlots) {
+        BinBlocks bb{};
+        int used = 0;
+        bb.nslots = (int)(nslots - k0 < kBinSlots ? nslots - k0 : kBinSlots);
+        for (int k = 0; k < bb.nslots; ++k) {
+            const int32_t* v = slots + 4 * (k0 + k);
+            int b = 0;
+            while (b < used && bb.M[b] != blocks[v[0]]) ++b;
+            if (b == used) bb.M[used++] = blocks[v[0]];
+            bb.block[k] = (signed char)b;
+            bb.c1[k] = (signed char)v[1];
+            bb.c2[k] = (signed char)v[2];
+            bb.sign[k] = (signed char)v[3];
+        }
+        hipLaunchKernelGGL(k_bin_blocks, dim3((unsigned)((nbands + nbw - 1) / nbw), (unsigned)nbands, (unsigned)used),
+                           dim3(256), 0, (hipStream_t)stream, bb, (int)(lmax + 1), ells, band_start, (int)nbands, wout, tin,
+                           (int)ncls, nbw, out);
+    }
     return check_launch("gm_bin_blocks");
 }
 

@@ -309,7 +309,7 @@ int gm_bin_block(const double* M, int64_t lmax, const int32_t* ells, const int32
 
 /* The same for every block of a binned coupling matrix, into its slots: slots holds (block, c1,
  * c2, sign) per slot, out[b1 ncls + c1][b2 ncls + c2] = sign x binned block (rows of nbands ncls).
- * blocks (device pointers) and slots are host arrays, at most 16 of each; other slots are left. */
+ * blocks (device pointers) and slots are host arrays; other slots are left. */
 int gm_bin_blocks(const double* const* blocks, int64_t nblocks, int64_t lmax, const int32_t* ells,
                   const int32_t* band_start, int64_t nbands, const double* wout, const double* tin,
                   int64_t ncls, const int32_t* slots, int64_t nslots, double* out, void* stream);
