@@ -48,7 +48,7 @@ SIGNATURES = {
     "gm_lat_syn_s_mixed": [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _i64, _p],
     "gm_lat2_chunks": [_i64, _i64],
     "gm_lat2_slots": [_i64, _i64],
-    "gm_lat2_polar_blocks": [_i64, _i64],
+    "gm_lat2_polar_size": [_i64, _i64, _i64, _i64],
     "gm_lat2_ana": [_p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p],
     "gm_lat2_finish": [_p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _i32, _i64, _p],
     "gm_lat2_prep": [_p, _p, _p, _p, _i64, _i64, _p, _p, _p],
@@ -102,7 +102,7 @@ SIGNATURES = {
     "gm_abi_version": [],
     "gm_last_error": [],
 }
-_RET_I64 = {"gm_lat2_chunks", "gm_lat2_slots", "gm_lat2_polar_blocks", "gm_bat_blocks", "gm_bat_stride", "gm_coupled_cell_noalloc_max_work", "gm_apodize_work_size", "gm_lat_ring_chunks", "gm_map_dots_work_size", "gm_lat_nchunks_mixed", "gm_table_size", "gm_lat_nchunks", "gm_cl_work_size"}
+_RET_I64 = {"gm_lat2_chunks", "gm_lat2_slots", "gm_lat2_polar_size", "gm_bat_blocks", "gm_bat_stride", "gm_coupled_cell_noalloc_max_work", "gm_apodize_work_size", "gm_lat_ring_chunks", "gm_map_dots_work_size", "gm_lat_nchunks_mixed", "gm_table_size", "gm_lat_nchunks", "gm_cl_work_size"}
 
 _lib = None
 

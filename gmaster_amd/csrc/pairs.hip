@@ -14,7 +14,15 @@
 // divided by s^2 at the end.  That is 6 FP64 operations per (degree, ring pair) where the
 // spin-2 recurrence on every ring takes 12.  The 1/s^2 amplifies rounding towards the
 // poles, so ring pairs with s^2 below the caller's split run the spin-2 recurrence instead
-// (the "polar" blocks of the same launch).
+// (the "polar" blocks of the same launch).  In the orders m < kLowOrders the amplified rounding is
+// not hidden by the rows themselves -- at m = 0 the spin-2 rows fall as s^2 towards the pole while
+// the rounding of their 1/s^2 terms grows as 1/s^2, at m >= 2 both stay alike -- and those orders
+// take the spin-0 rows in the belt only (s^2 >= 5/9).
+// Syntheses of a field with power at l <= m + 10, Nside 64, rms error against long double over that of
+// the spin-2 recurrence on every ring: orders 0 - 3 3.4 when split at 1/64 like the others, 1.0 with
+// the belt alone; orders 4 - 7 1.4, 1.0; orders 8 - 15 (split at 1/64) 1.0; spectra as (l + 1)^-2
+// 1.5, 1.0; 1.1, 1.0; 1.04.  The low orders' caps cost 1% of a transform (three iterations at
+// Nside 1024 17.8 -> 18.0 ms, a synthesis at 2048 17.2 -> 17.3 ms, an analysis at 512 308 -> 311 us).
 //
 // Analysis reduction over rings: every degree each lane writes its 2K partial sums to LDS as
 // 16-byte words, and once per 8 degrees the workgroup's threads sum them (T 4K reads), so the
@@ -56,6 +64,14 @@ __device__ inline int slot_ring(int nside, int j) {
     const int u = (j + 1) / 2;
     return (j & 1) ? 2 * nside - 1 - u : 2 * nside - 1 + u;
 }
+
+// Orders m < n take the spin-0 rows for the ring pairs below j, their other ring slots in nb polar
+// blocks.
+constexpr int kLowOrders = 8;
+struct Low {
+    int n, j, nb;
+    __device__ int pairs(int m, int jend) const { return m < n ? min(j, jend) : jend; }
+};
 
 struct Tables {
     const double* __restrict__ alpha;
@@ -305,30 +321,35 @@ __device__ __forceinline__ void with_sets(int n, F&& body) {
     body(Int<RMAX>{});
 }
 
-// Grid (1-D): npol polar blocks (order-major), then nblk blocks of ring pairs per order, over
-// the ring pairs jbeg .. jend - 1.
+// Grid (1-D): npol polar blocks (order-major; low.nb of each low order, nbp of the others), then
+// nblk blocks of ring pairs per order, over the ring pairs jbeg .. jend - 1.  ppart: nbp slots of
+// ptsize entries, then low.nb slots of the low orders'.
 template <int K, int R, int NW, bool SP2, int RP>
 __global__ __launch_bounds__(64 * NW, 2) void k_ana_pairs(const double2* __restrict__ spec, int64_t ld, int64_t smap,
                                                           int nside, int Lm, Tables tab, int jbeg, int jend, int nblk,
                                                           double* __restrict__ partial, Tables pol, int pbeg, int nbp,
-                                                          int npol, double* __restrict__ ppart, int64_t ptsize) {
+                                                          int npol, Low low, double* __restrict__ ppart,
+                                                          int64_t ptsize) {
     constexpr int T = 64 * NW;
     __shared__ double2 lds[kDeg * K * T];
     int b = blockIdx.x;
     if constexpr (SP2) {
         if (b < npol) {
-            const int m = b / nbp, c = b % nbp;
-            const int j0 = pbeg + c * T * RP;
+            const int bl = b - low.n * low.nb;
+            const bool lo = bl < 0;
+            const int m = lo ? b / low.nb : low.n + bl / nbp, c = lo ? b % low.nb : bl % nbp;
+            const int j0 = (lo ? 2 * low.j - 1 : pbeg) + c * T * RP;
             const int na = pol.nact[m];
             if (j0 >= na) return;
-            double* part = ppart + ((int64_t)c * ptsize + table_base(m, pol.L) - m) * 4;
+            const int64_t slot = lo ? nbp * ptsize + c * table_base(low.n, pol.L) : c * ptsize;
+            double* part = ppart + (slot + table_base(m, pol.L) - m) * 4;
             ana_body<K, RP, NW, SP2, true>(spec, ld, smap, nside, Lm, 2, pol, m, j0, na, part, lds);
             return;
         }
         b -= npol;
     }
     const int m = b / nblk, c = b % nblk;
-    const int jhi = min(tab.nact[m], jend);
+    const int jhi = min(tab.nact[m], low.pairs(m, jend));
     const Split sp(jhi - jbeg, T, R);
     const int n = min(sp.spb, sp.total - c * sp.spb);
     if (n <= 0) return;
@@ -513,18 +534,20 @@ __device__ __forceinline__ void syn_body(const double2* __restrict__ cf, int nsi
 template <int K, int R, int NW, bool SP2, int RP>
 __global__ __launch_bounds__(64 * NW, 2) void k_syn_pairs(const double2* __restrict__ coef, int nside, int Lm, Tables tab,
                                                           int jend, int nblk, const double2* __restrict__ pcoef,
-                                                          Tables pol, int nbp, int npol, double2* __restrict__ spec,
-                                                          int64_t ld, int64_t smap) {
+                                                          Tables pol, int nbp, int npol, Low low,
+                                                          double2* __restrict__ spec, int64_t ld, int64_t smap) {
     constexpr int T = 64 * NW;
     __shared__ __align__(16) double2 st[NW * stage_words(K)];
     int b = blockIdx.x;
     if constexpr (SP2) {
         const int npair = nblk * Lm;
         if (b < npol || b >= npol + npair) {
-            if (b >= npol) b -= npair;
-            const int m = b / nbp, c = b % nbp;
-            const int j0 = 2 * jend - 1 + c * T * RP;
-            const bool any = (int64_t)m * nbp < npol;
+            const bool any = b < npol;
+            if (!any) b -= npair;
+            const int bl = b - low.n * low.nb;
+            const bool lo = bl < 0;
+            const int m = lo ? b / low.nb : low.n + bl / nbp, c = lo ? b % low.nb : bl % nbp;
+            const int j0 = 2 * (lo ? low.j : jend) - 1 + c * T * RP;
             const double2* cf = pcoef + (table_base(m, pol.L) - m) * 2;
             syn_body<K, RP, NW, SP2, true>(cf, nside, Lm, 2, pol, m, j0, any ? pol.nact[m] : 0, 4 * nside - 1, spec, ld,
                                            smap, st);
@@ -533,6 +556,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_syn_pairs(const double2* __restr
         b -= npol;
     }
     const int m = b / nblk, c = b % nblk;
+    jend = low.pairs(m, jend);
     const int jhi = min(tab.nact[m], jend);
     const double2* cf = coef + (table_base(m, tab.L) - m) * K;
     const Split sp(jhi, T, R);
@@ -594,7 +618,7 @@ constexpr int kFin = 256;
 __global__ __launch_bounds__(kFin) void k_finish_2(const double* __restrict__ partial, const double* __restrict__ ppart,
                                                    int T, int RMAX, int jbeg, int jend, int jsplit,
                                                    const int* __restrict__ nact,
-                                                   const double* __restrict__ P, int nbp, int CHP, int mpol,
+                                                   const double* __restrict__ P, int nbp, int CHP, int mpol, Low low,
                                                    const int* __restrict__ nact2, const double* __restrict__ P2, int Lm,
                                                    int64_t ptsize, double2* __restrict__ ae, double2* __restrict__ ab,
                                                    int mode) {
@@ -602,7 +626,7 @@ __global__ __launch_bounds__(kFin) void k_finish_2(const double* __restrict__ pa
     const int Lt = Lm + 2;
     const int m = blockIdx.y, lb = m + blockIdx.x * kFin;
     if (lb >= Lm) return;
-    const int nu = Split(min(nact[m], jend) - jbeg, T, RMAX).blocks();
+    const int nu = Split(min(nact[m], low.pairs(m, jend)) - jbeg, T, RMAX).blocks();
     const int64_t ts = table_size(Lt), pb = table_base(m, Lt) - m;
     const double2* p2 = reinterpret_cast<const double2*>(partial);
     for (int h = threadIdx.x; h < kFin + 4; h += kFin) {
@@ -638,11 +662,13 @@ __global__ __launch_bounds__(kFin) void k_finish_2(const double* __restrict__ pa
     double2 E = make_double2(-(wq.x - xu.y), -(wq.y + xu.x));
     double2 B = make_double2(-xq.y - wu.x, xq.x - wu.y);
     if (m < mpol && jbeg == 0 && l >= 2) {
-        const int np = min(nbp, (nact2[m] - (2 * jsplit - 1) + CHP - 1) / CHP);
+        const bool lo = m < low.n;
+        const int np = min(lo ? low.nb : nbp, (nact2[m] - (2 * (lo ? low.j : jsplit) - 1) + CHP - 1) / CHP);
         const int64_t qb = table_base(m, Lm) - m;
+        const int64_t slots = lo ? nbp * ptsize : 0, stride = lo ? table_base(low.n, Lm) : ptsize;
         double2 d = z, mi = z;
         for (int k = 0; k < np; ++k) {
-            const double2* p = reinterpret_cast<const double2*>(ppart) + ((int64_t)k * ptsize + qb + l) * 2;
+            const double2* p = reinterpret_cast<const double2*>(ppart) + (slots + k * stride + qb + l) * 2;
             d = cadd(d, p[0]);
             mi = cadd(mi, p[1]);
         }
@@ -764,20 +790,28 @@ Shape pair_shape(int64_t nside, int K, bool sp2, bool syn) {
 int npolar_slots(int64_t nside, int64_t jsplit) { return (int)(4 * nside - 1 - (2 * jsplit - 1)); }
 constexpr int kRP = 2;
 
+// Polar blocks of CHP ring slots beyond the ring pairs below j.
+int polar_blocks(int64_t nside, int64_t j, int CHP) { return (npolar_slots(nside, j) + CHP - 1) / CHP; }
+
+Low low_orders(int64_t nside, int64_t lmax, int64_t jsplit, int CHP) {
+    const int64_t belt = nside + 1, j = belt < jsplit ? belt : jsplit;
+    return Low{(int)(lmax + 1 < kLowOrders ? lmax + 1 : kLowOrders), (int)j, polar_blocks(nside, j, CHP)};
+}
+
 }  // namespace
 
 int pairs_chunk(int64_t nside, int K) { return pair_shape(nside, K, false, false).CH; }
 
 template <int K, bool SP2>
 int launch_ana(const char* name, const double2* spec, int64_t ld, int64_t smap, int nside, int Lm, const Tables& tab,
-               int jbeg, int jend, int nblk, double* partial, const Tables& pol, int pbeg, int nbp, int npol,
+               int jbeg, int jend, int nblk, double* partial, const Tables& pol, int pbeg, int nbp, int npol, const Low& low,
                double* ppart, int64_t ptsize, hipStream_t st) {
     const Shape s = pair_shape(nside, K, SP2, false);
     const dim3 grid((unsigned)(npol + nblk * Lm)), block(64 * s.NW);
 #define GM_GO(RR, WW)                                                                                                  \
     if (s.R == RR && s.NW == WW) {                                                                                     \
         hipLaunchKernelGGL((k_ana_pairs<K, RR, WW, SP2, kRP>), grid, block, 0, st, spec, ld, smap, nside, Lm, tab, jbeg, \
-                           jend, nblk, partial, pol, pbeg, nbp, npol, ppart, ptsize);                                      \
+                           jend, nblk, partial, pol, pbeg, nbp, npol, low, ppart, ptsize);                                 \
         return check_launch(name);                                                                                     \
     }
     GM_GO(2, 1)
@@ -791,14 +825,14 @@ int launch_ana(const char* name, const double2* spec, int64_t ld, int64_t smap, 
 
 template <int K, bool SP2>
 int launch_syn(const char* name, const double2* coef, int nside, int Lm, const Tables& tab, int jend, int nblk,
-               const double2* pcoef, const Tables& pol, int nbp, int npol, int nzero, double2* spec, int64_t ld,
-               int64_t smap, hipStream_t st) {
+               const double2* pcoef, const Tables& pol, int nbp, int npol, int nzero, const Low& low, double2* spec,
+               int64_t ld, int64_t smap, hipStream_t st) {
     const Shape s = pair_shape(nside, K, SP2, true);
     const dim3 grid((unsigned)(npol + nblk * Lm + nzero)), block(64 * s.NW);
 #define GM_GO(RR, WW)                                                                                                \
     if (s.R == RR && s.NW == WW) {                                                                                   \
         hipLaunchKernelGGL((k_syn_pairs<K, RR, WW, SP2, kRP>), grid, block, 0, st, coef, nside, Lm, tab, jend, nblk, pcoef, \
-                           pol, nbp, npol, spec, ld, smap);                                                          \
+                           pol, nbp, npol, low, spec, ld, smap);                                                     \
         return check_launch(name);                                                                                   \
     }
     GM_GO(1, 2)
@@ -818,9 +852,9 @@ int ana_pairs_s0(const char* name, const double* spec, int K, int64_t ld, int64_
     hipStream_t st = (hipStream_t)stream;
     if (K == 1)
         return launch_ana<1, false>(name, sp, ld, smap, (int)nside, (int)L, tab, jbeg, jend, nblk, partial, tab, 0,
-                                    1, 0, nullptr, 0, st);
+                                    1, 0, Low{0, 0, 1}, nullptr, 0, st);
     return launch_ana<2, false>(name, sp, ld, smap, (int)nside, (int)L, tab, jbeg, jend, nblk, partial, tab, 0, 1, 0,
-                                nullptr, 0, st);
+                                Low{0, 0, 1}, nullptr, 0, st);
 }
 
 int finish_pairs_s0(const char* name, const double* partial, int K, int64_t nside, int64_t L, const int32_t* nact,
@@ -842,10 +876,10 @@ int syn_pairs_s0(const char* name, const double* coef, int K, int64_t nside, int
     const int CH = pair_shape(nside, K, false, true).CH;
     const int nblk = (int)((2 * nside + CH - 1) / CH);
     if (K == 1)
-        return launch_syn<1, false>(name, cf, (int)nside, (int)L, tab, (int)(2 * nside), nblk, nullptr, tab, 1, 0, 0, sp, ld,
-                                    smap, st);
-    return launch_syn<2, false>(name, cf, (int)nside, (int)L, tab, (int)(2 * nside), nblk, nullptr, tab, 1, 0, 0, sp, ld,
-                                smap, st);
+        return launch_syn<1, false>(name, cf, (int)nside, (int)L, tab, (int)(2 * nside), nblk, nullptr, tab, 1, 0, 0,
+                                    Low{0, 0, 1}, sp, ld, smap, st);
+    return launch_syn<2, false>(name, cf, (int)nside, (int)L, tab, (int)(2 * nside), nblk, nullptr, tab, 1, 0, 0,
+                                Low{0, 0, 1}, sp, ld, smap, st);
 }
 
 }  // namespace gm
@@ -857,7 +891,8 @@ int check_2(const char* name, int64_t nside, int64_t lmax, int64_t jsplit, int64
     if (nside < 1 || (nside & (nside - 1)) || nside > 8192) return fail(GM_E_ARG, "%s: bad nside", name);
     if (lmax < 2 || lmax > 24 * nside) return fail(GM_E_ARG, "%s: bad lmax %lld", name, (long long)lmax);
     if (jsplit < 1 || jsplit > 2 * nside) return fail(GM_E_ARG, "%s: jsplit outside [1, 2 nside]", name);
-    if (mpol < 0 || mpol > lmax + 1) return fail(GM_E_ARG, "%s: mpol outside [0, lmax + 1]", name);
+    const int64_t low = lmax + 1 < kLowOrders ? lmax + 1 : kLowOrders;
+    if (mpol < low || mpol > lmax + 1) return fail(GM_E_ARG, "%s: mpol outside [min(%d, lmax + 1), lmax + 1]", name, kLowOrders);
     return GM_OK;
 }
 constexpr int kSlots = 4;
@@ -874,10 +909,11 @@ extern "C" int64_t gm_lat2_slots(int64_t nside, int64_t jsplit) {
     return nside <= 4096 || n <= kSlots ? n : kSlots;
 }
 
-extern "C" int64_t gm_lat2_polar_blocks(int64_t nside, int64_t jsplit) {
-    if (nside < 1 || jsplit < 1 || jsplit > 2 * nside) return -1;
-    const int chp = 64 * pair_shape(nside, 2, true, false).NW * kRP;
-    return (npolar_slots(nside, jsplit) + chp - 1) / chp;
+extern "C" int64_t gm_lat2_polar_size(int64_t nside, int64_t lmax, int64_t jsplit, int64_t mpol) {
+    if (check_2("gm_lat2_polar_size", nside, lmax, jsplit, mpol)) return -1;
+    const int CHP = 64 * pair_shape(nside, 2, true, false).NW * kRP;
+    const Low low = low_orders(nside, lmax, jsplit, CHP);
+    return 4 * (polar_blocks(nside, jsplit, CHP) * table_base(mpol, lmax + 1) + low.nb * table_base(low.n, lmax + 1));
 }
 
 extern "C" int gm_lat2_ana(const double* spec, int64_t ld, int64_t nside, int64_t lmax, int64_t jsplit, int64_t mpol,
@@ -886,8 +922,7 @@ extern "C" int gm_lat2_ana(const double* spec, int64_t ld, int64_t nside, int64_
                            const int32_t* nact2, double* part, double* ppart, int64_t chunk0, void* stream) {
     const char* name = "gm_lat2_ana";
     if (int e = check_2(name, nside, lmax, jsplit, mpol)) return e;
-    if (!spec || !alpha || !smant || !sexp || !nact || !part) return fail(GM_E_ARG, "%s: null pointer", name);
-    if (mpol > 0 && (!alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2 || !ppart))
+    if (!spec || !alpha || !smant || !sexp || !nact || !part || !alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2 || !ppart)
         return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t Lm = lmax + 1;
     if (ld < 2 * Lm - 1) return fail(GM_E_SHAPE, "%s: ld < 2 lmax + 1", name);
@@ -896,12 +931,13 @@ extern "C" int gm_lat2_ana(const double* spec, int64_t ld, int64_t nside, int64_
     const int nblk = (int)(chunks - chunk0 < slots ? chunks - chunk0 : slots);
     const Tables tab{alpha, nullptr, smant, sexp, nact, (int)Lm + 2};
     const Tables pol{alpha2, gamma2, smant2, sexp2, nact2, (int)Lm};
-    const int nbp = (int)gm_lat2_polar_blocks(nside, jsplit);
-    const int npol = chunk0 == 0 ? (int)(mpol * nbp) : 0;
-    const int CH = pair_shape(nside, 2, true, false).CH;
+    const Shape s = pair_shape(nside, 2, true, false);
+    const int CH = s.CH, CHP = 64 * s.NW * kRP, nbp = polar_blocks(nside, jsplit, CHP);
+    const Low low = low_orders(nside, lmax, jsplit, CHP);
+    const int npol = chunk0 == 0 ? low.n * low.nb + ((int)mpol - low.n) * nbp : 0;
     const int jbeg = (int)chunk0 * CH, jend = jbeg + nblk * CH < jsplit ? jbeg + nblk * CH : (int)jsplit;
     return launch_ana<2, true>(name, reinterpret_cast<const double2*>(spec), ld, 0, (int)nside, (int)Lm, tab, jbeg, jend,
-                               nblk, part, pol, (int)(2 * jsplit - 1), nbp > 0 ? nbp : 1, npol, ppart,
+                               nblk, part, pol, (int)(2 * jsplit - 1), nbp, npol, low, ppart,
                                table_base(mpol, Lm), (hipStream_t)stream);
 }
 
@@ -911,7 +947,7 @@ extern "C" int gm_lat2_finish(const double* part, const double* ppart, int64_t n
     const char* name = "gm_lat2_finish";
     if (int e = check_2(name, nside, lmax, jsplit, mpol)) return e;
     if (mode < 0 || mode > 2 || chunk0 < 0) return fail(GM_E_ARG, "%s: bad mode / chunk0", name);
-    if (!part || !nact || !P || !alm_e || !alm_b || (mpol > 0 && (!ppart || !nact2 || !P2)))
+    if (!part || !nact || !P || !alm_e || !alm_b || !ppart || !nact2 || !P2)
         return fail(GM_E_ARG, "%s: null pointer", name);
     const int Lm = (int)lmax + 1;
     const Shape s = pair_shape(nside, 2, true, false);
@@ -919,7 +955,8 @@ extern "C" int gm_lat2_finish(const double* part, const double* ppart, int64_t n
     const int64_t end = (chunk0 + gm_lat2_slots(nside, jsplit)) * s.CH;
     hipLaunchKernelGGL(k_finish_2, dim3((Lm + kFin - 1) / kFin, Lm), dim3(kFin), 0, (hipStream_t)stream, part, ppart, T, s.R,
                        (int)chunk0 * s.CH, (int)(end < jsplit ? end : jsplit), (int)jsplit, nact, P,
-                       (int)gm_lat2_polar_blocks(nside, jsplit), CHP, (int)mpol, nact2, P2, Lm, table_base(mpol, Lm),
+                       polar_blocks(nside, jsplit, CHP), CHP, (int)mpol, low_orders(nside, lmax, jsplit, CHP), nact2, P2, Lm,
+                       table_base(mpol, Lm),
                        reinterpret_cast<double2*>(alm_e), reinterpret_cast<double2*>(alm_b), mode);
     return check_launch(name);
 }
@@ -928,7 +965,7 @@ extern "C" int gm_lat2_prep(const double* alm_e, const double* alm_b, const doub
                             int64_t mpol, double* coef, double* pcoef, void* stream) {
     const char* name = "gm_lat2_prep";
     if (int e = check_2(name, 8192, lmax, 1, mpol)) return e;
-    if (!alm_e || !alm_b || !P || !coef || (mpol > 0 && (!P2 || !pcoef))) return fail(GM_E_ARG, "%s: null pointer", name);
+    if (!alm_e || !alm_b || !P || !coef || !P2 || !pcoef) return fail(GM_E_ARG, "%s: null pointer", name);
     const int Lm = (int)lmax + 1;
     hipLaunchKernelGGL(k_prep_2, dim3((Lm + 2 + GM_TABLE_PAD + kFin - 1) / kFin, Lm), dim3(kFin), 0, (hipStream_t)stream,
                        reinterpret_cast<const double2*>(alm_e), reinterpret_cast<const double2*>(alm_b), P, P2, Lm,
@@ -942,8 +979,7 @@ extern "C" int gm_lat2_syn(const double* coef, const double* pcoef, int64_t nsid
                            const int32_t* sexp2, const int32_t* nact2, double* spec, int64_t ld, void* stream) {
     const char* name = "gm_lat2_syn";
     if (int e = check_2(name, nside, lmax, jsplit, mpol)) return e;
-    if (!coef || !alpha || !smant || !sexp || !nact || !spec) return fail(GM_E_ARG, "%s: null pointer", name);
-    if (mpol > 0 && (!pcoef || !alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2))
+    if (!coef || !alpha || !smant || !sexp || !nact || !spec || !pcoef || !alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2)
         return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t Lm = lmax + 1;
     if (ld < 2 * Lm - 1) return fail(GM_E_SHAPE, "%s: ld < 2 lmax + 1", name);
@@ -951,8 +987,10 @@ extern "C" int gm_lat2_syn(const double* coef, const double* pcoef, int64_t nsid
     const Tables pol{alpha2, gamma2, smant2, sexp2, nact2, (int)Lm};
     const Shape s = pair_shape(nside, 2, true, true);
     const int CH = s.CH, chp = 64 * s.NW * kRP;
-    const int nblk = (int)((jsplit + CH - 1) / CH), nbp = (npolar_slots(nside, jsplit) + chp - 1) / chp;
+    const int nblk = (int)((jsplit + CH - 1) / CH), nbp = polar_blocks(nside, jsplit, chp);
+    const Low low = low_orders(nside, lmax, jsplit, chp);
+    const int npol = low.n * low.nb + ((int)mpol - low.n) * nbp;
     return launch_syn<2, true>(name, reinterpret_cast<const double2*>(coef), (int)nside, (int)Lm, tab, (int)jsplit, nblk,
-                               reinterpret_cast<const double2*>(pcoef), pol, nbp > 0 ? nbp : 1, (int)(mpol * nbp),
-                               (int)((Lm - mpol) * nbp), reinterpret_cast<double2*>(spec), ld, 0, (hipStream_t)stream);
+                               reinterpret_cast<const double2*>(pcoef), pol, nbp, npol, (int)((Lm - mpol) * nbp), low,
+                               reinterpret_cast<double2*>(spec), ld, 0, (hipStream_t)stream);
 }

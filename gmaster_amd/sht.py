@@ -159,9 +159,11 @@ def plan(nside, lmax, spin, device=None, polar_skip=True):
 # Ring pairs with sin^2(theta) below this run the spin-2 recurrence itself; the others the
 # spin-0 rows with weights 1/sin^2, which amplify rounding by up to this bound's inverse.  The
 # polar blocks cost four times a ring pair's: 1/32 -> 1/64 measured 18.6 -> 17.9 ms for map2alm
-# with three iterations at Nside 1024 and 42.7 -> 40.7 ms for a T+P run, the error against exact
-# sums unchanged from Nside 512 on (1.4e-14, 2.8e-13) and 1 - 1.4 of 2e-15 at Nside 64.
+# with three iterations at Nside 1024 and 42.7 -> 40.7 ms for a T+P run.  The amplified rounding
+# shows in the lowest orders of smooth fields; below LOW_ORDERS the kernels take the spin-0
+# rows in the belt only (csrc/pairs.hip has the errors).
 PAIR_SIN2 = 1.0 / 64.0
+LOW_ORDERS = 8
 
 
 @dataclass
@@ -174,10 +176,10 @@ class Plan2:
     pol: Plan              # spin-2 tables (polar rings)
     nact: torch.Tensor     # ring pairs visited by order m
     jsplit: int            # first ring pair of the polar part
-    mpol: int              # orders that reach the polar rings
+    mpol: int              # orders that reach the polar rings, LOW_ORDERS at least
     nslots: int
     nchunks: int
-    nbp: int               # polar blocks per order
+    polar_size: int        # doubles of the polar blocks' partial sums
     tsize: int             # entries of the spin-0 tables
     ptsize: int            # entries of the spin-2 tables of the orders m < mpol
 
@@ -194,13 +196,14 @@ def plan2(nside, lmax, device=None, polar_skip=True):
     L = lmax + 1
     jsplit = _split_at(nside, PAIR_SIN2)
     mpol = int(np.count_nonzero(_nactive(nside, lmax, 2, polar_skip) > 2 * jsplit - 1))
+    mpol = max(mpol, min(LOW_ORDERS, L))
     p = Plan2(
         nside=nside, lmax=lmax, device=device, tab=plan(nside, lmax + 2, 0, device, polar_skip),
         pol=plan(nside, lmax, 2, device, polar_skip),
         nact=torch.as_tensor(_nactive_pairs(nside, lmax, polar_skip), dtype=torch.int32, device=device),
         jsplit=jsplit, mpol=mpol, nslots=int(_lib.query("gm_lat2_slots", nside, jsplit)),
         nchunks=int(_lib.query("gm_lat2_chunks", nside, jsplit)),
-        nbp=int(_lib.query("gm_lat2_polar_blocks", nside, jsplit)),
+        polar_size=int(_lib.query("gm_lat2_polar_size", nside, lmax, jsplit, mpol)),
         tsize=int(_lib.query("gm_table_size", lmax + 2)), ptsize=mpol * (L + 8) - mpol * (mpol - 1) // 2,
     )
     _PLANS[key] = p
@@ -418,7 +421,7 @@ def _analysis_2(p, spec, ae, ab, mode):
     """FP64 spin-2 analysis on the spin-0 rows (polar rings: the spin-2 recurrence)."""
     st = _lib.stream_ptr(p.device)
     part = torch.empty(p.nslots * p.tsize * 4, dtype=torch.float64, device=p.device)
-    ppart = torch.empty(p.nbp * p.ptsize * 4, dtype=torch.float64, device=p.device) if p.mpol else None
+    ppart = torch.empty(p.polar_size, dtype=torch.float64, device=p.device)
     t, q = p.tab, p.pol
     for c0 in range(0, p.nchunks, p.nslots):
         md = int(mode) if c0 == 0 else (1 if mode == 1 else 2)
@@ -433,7 +436,7 @@ def _analysis_2(p, spec, ae, ab, mode):
 def _synthesis_2(p, ae, ab, spec):
     st = _lib.stream_ptr(p.device)
     coef = torch.empty(p.tsize * 2, dtype=torch.complex128, device=p.device)
-    pcoef = torch.empty(p.ptsize * 2, dtype=torch.complex128, device=p.device) if p.mpol else None
+    pcoef = torch.empty(p.ptsize * 2, dtype=torch.complex128, device=p.device)
     t, q = p.tab, p.pol
     _lib.call("gm_lat2_prep", _lib.ptr(ae), _lib.ptr(ab), _lib.ptr(t.P), _lib.ptr(q.P), p.lmax, p.mpol, _lib.ptr(coef),
               _lib.ptr(pcoef), st)

@@ -156,19 +156,19 @@ int gm_lat_syn_s(const double* coef, int64_t nside, int64_t lmax, int64_t spin, 
                  const int32_t* nactive, double* spec, int64_t ld, void* stream);
 
 /* ---------------------------------------------------------------- spin 2 on spin-0 rows, FP64
- * The spin-2 transforms of ring pairs j < jsplit through the spin-0 rows with weights
- * 1/sin^2 (tables of lmax + 2, nactive in ring pairs), the rings beyond (slots >= 2 jsplit - 1)
- * through the spin-2 recurrence (tables of lmax, nactive2 in ring slots; orders m < mpol, the
- * others do not reach them).  No counterpart in the reference, which runs a spin-2 recurrence
- * on every ring (gmaster/_native/cuda/march_v2.cu:553-556).
+ * The spin-2 transforms of ring pairs j < jsplit (j <= nside, the belt, in the orders m < 8)
+ * through the spin-0 rows with weights 1/sin^2 (tables of lmax + 2, nactive in ring pairs), the
+ * rings beyond through the spin-2 recurrence (tables of lmax, nactive2 in ring slots; orders
+ * m < mpol, the others do not reach them; mpol >= min(8, lmax + 1)).  No counterpart in the
+ * reference, which runs a spin-2 recurrence on every ring (gmaster/_native/cuda/march_v2.cu:553-556).
  *   part   gm_lat2_slots x gm_table_size(lmax + 2) x 4 double
- *   ppart  gm_lat2_polar_blocks x (mpol (lmax + 9) - mpol (mpol - 1) / 2) x 4 double
- *   coef   gm_table_size(lmax + 2) x 4 double; pcoef: one block's entries of ppart
+ *   ppart  gm_lat2_polar_size double
+ *   coef   gm_table_size(lmax + 2) x 4 double; pcoef (mpol (lmax + 9) - mpol (mpol - 1) / 2) x 4 double
  * Analysis passes start at chunk0 = 0, slots, 2 slots, ... below gm_lat2_chunks; mode 0 stores,
  * 1 subtracts, 2 adds. */
 int64_t gm_lat2_chunks(int64_t nside, int64_t jsplit);
 int64_t gm_lat2_slots(int64_t nside, int64_t jsplit);
-int64_t gm_lat2_polar_blocks(int64_t nside, int64_t jsplit);
+int64_t gm_lat2_polar_size(int64_t nside, int64_t lmax, int64_t jsplit, int64_t mpol);
 int gm_lat2_ana(const double* spec, int64_t ld, int64_t nside, int64_t lmax, int64_t jsplit, int64_t mpol,
                 const double* alpha, const double* seed_mant, const int32_t* seed_exp, const int32_t* nactive,
                 const double* alpha2, const double* gamma2, const double* seed_mant2, const int32_t* seed_exp2,
