@@ -680,6 +680,7 @@ __global__ __launch_bounds__(kFin) void k_finish_2(const double* __restrict__ pa
         E = make_double2(E.x - 0.5 * (plus.x + mn.x), E.y - 0.5 * (plus.y + mn.y));
         B = make_double2(B.x - 0.5 * (plus.y - mn.y), B.y + 0.5 * (plus.x - mn.x));
     }
+    if (l < 2) E = B = z;  // not zero times a sum that need not be finite
     const int64_t ia = alm_index(l, m, Lm - 1);
     ae[ia] = mode == 1 ? csub(ae[ia], E) : mode == 2 ? cadd(ae[ia], E) : E;
     ab[ia] = mode == 1 ? csub(ab[ia], B) : mode == 2 ? cadd(ab[ia], B) : B;
