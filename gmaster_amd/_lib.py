@@ -96,13 +96,14 @@ SIGNATURES = {
     "gm_gauss_draws": [ctypes.c_uint64, _i64, _i64, _p, _p],
     "gm_table_size": [_i64],
     "gm_lat_nchunks": [_i64, _i64],
+    "gm_lat_slots_s0": [_i64],
     "gm_lat_nchunks_mixed": [_i64, _i64, _i64],
     "gm_lat_ring_chunks": [_i64, _i64, _i64, _i64],
     "gm_cl_work_size": [_i64, _i64],
     "gm_abi_version": [],
     "gm_last_error": [],
 }
-_RET_I64 = {"gm_lat2_chunks", "gm_lat2_slots", "gm_lat2_polar_size", "gm_bat_blocks", "gm_bat_stride", "gm_coupled_cell_noalloc_max_work", "gm_apodize_work_size", "gm_lat_ring_chunks", "gm_map_dots_work_size", "gm_lat_nchunks_mixed", "gm_table_size", "gm_lat_nchunks", "gm_cl_work_size"}
+_RET_I64 = {"gm_lat_slots_s0", "gm_lat2_chunks", "gm_lat2_slots", "gm_lat2_polar_size", "gm_bat_blocks", "gm_bat_stride", "gm_coupled_cell_noalloc_max_work", "gm_apodize_work_size", "gm_lat_ring_chunks", "gm_map_dots_work_size", "gm_lat_nchunks_mixed", "gm_table_size", "gm_lat_nchunks", "gm_cl_work_size"}
 
 _lib = None
 

@@ -948,6 +948,19 @@ int check_config(const char* name, const LatConfig& cfg, int large_r) {
     return GM_OK;
 }
 
+// The ring pairs jbeg .. jend - 1 of an FP64 spin-0 pass (its chunks'), which the pair kernels
+// cover in slots of their own size.
+void pass_pairs(const LatConfig& cfg, int64_t nside, int64_t chunk0, int& jbeg, int& jend) {
+    const int64_t end = (chunk0 + cfg.nslots) * cfg.CH;
+    jbeg = (int)(chunk0 * cfg.CH);
+    jend = (int)(end < 2 * nside ? end : 2 * nside);
+}
+
+int pass_slots(int64_t nside, int jbeg, int jend) {
+    const int CH = pairs_chunk(nside);
+    return (jend - jbeg + CH - 1) / CH;
+}
+
 int check_lat(int64_t nside, int64_t lmax, int64_t spin) {
     if (nside < 1 || (nside & (nside - 1))) return fail(GM_E_ARG, "nside must be a power of 2");
     if (nside > 8192) return fail(GM_E_UNSUPPORTED, "nside > 8192 not supported");
@@ -964,6 +977,19 @@ using namespace gm;
 extern "C" int64_t gm_table_size(int64_t lmax) { return table_size(lmax + 1); }
 
 extern "C" int64_t gm_lat_nchunks(int64_t nside, int64_t spin) { return lat_config(nside, spin).nslots; }
+
+extern "C" int64_t gm_lat_slots_s0(int64_t nside) {
+    if (check_lat(nside, 0, 0)) return -1;
+    const LatConfig cfg = lat_config(nside, 0);
+    int64_t slots = 0;
+    for (int64_t c0 = 0; c0 < cfg.nchunks; c0 += cfg.nslots) {
+        int jbeg, jend;
+        pass_pairs(cfg, nside, c0, jbeg, jend);
+        const int64_t n = pass_slots(nside, jbeg, jend);
+        if (n > slots) slots = n;
+    }
+    return slots;
+}
 
 extern "C" int64_t gm_lat_nchunks_mixed(int64_t nside, int64_t spin, int64_t nmaps) {
     return lat_config(nside, spin, true, (int)nmaps).nslots;
@@ -1003,14 +1029,6 @@ int check_pass(const char* name, const LatConfig& cfg, int64_t nchunks, int64_t 
     if (chunk0 < 0 || chunk0 >= cfg.nchunks || chunk0 % cfg.nslots)
         return fail(GM_E_ARG, "%s: chunk0 %lld is not a pass start below %d", name, (long long)chunk0, cfg.nchunks);
     return GM_OK;
-}
-
-// The ring pairs jbeg .. jend - 1 of an FP64 spin-0 pass (its chunks'), which the pair kernels
-// cover in slots of their own size.
-void pass_pairs(const LatConfig& cfg, int64_t nside, int64_t chunk0, int& jbeg, int& jend) {
-    const int64_t end = (chunk0 + cfg.nslots) * cfg.CH;
-    jbeg = (int)(chunk0 * cfg.CH);
-    jend = (int)(end < 2 * nside ? end : 2 * nside);
 }
 
 int launch_ana_s0_mixed(const char* name, const double* spec, int64_t nmaps, int64_t ld, int64_t smap, int64_t nside,
@@ -1176,7 +1194,7 @@ extern "C" int gm_lat_ana_s0(const double* spec, int64_t nmaps, int64_t ld, int6
     if (int e = check_pass(name, cfg, nchunks, chunk0)) return e;
     int jbeg, jend;
     pass_pairs(cfg, nside, chunk0, jbeg, jend);
-    const int CH = pairs_chunk(nside, (int)nmaps), nblk = (jend - jbeg + CH - 1) / CH;
+    const int nblk = pass_slots(nside, jbeg, jend);
     if (nblk > cfg.nslots) return fail(GM_E_LAUNCH, "%s: %d workgroups for %d partial slots", name, nblk, cfg.nslots);
     return ana_pairs_s0(name, spec, (int)nmaps, ld, smap, nside, lmax + 1, alpha, seed_mant, seed_exp, nactive, partial,
                         jbeg, jend, nblk, stream);

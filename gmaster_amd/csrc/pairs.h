@@ -5,8 +5,8 @@
 
 namespace gm {
 
-// Ring pairs per workgroup (and per partial slot) of the FP64 spin-0 analysis of K maps.
-int pairs_chunk(int64_t nside, int K);
+// Ring pairs per workgroup (and per partial slot) of the FP64 spin-0 analyses.
+int pairs_chunk(int64_t nside);
 
 // Ring pairs jbeg .. jend - 1 in nblk workgroups per order, one partial slot each.
 int ana_pairs_s0(const char* name, const double* spec, int K, int64_t ld, int64_t smap, int64_t nside, int64_t L,

@@ -801,7 +801,7 @@ Low low_orders(int64_t nside, int64_t lmax, int64_t jsplit, int CHP) {
 
 }  // namespace
 
-int pairs_chunk(int64_t nside, int K) { return pair_shape(nside, K, false, false).CH; }
+int pairs_chunk(int64_t nside) { return pair_shape(nside, 1, false, false).CH; }
 
 template <int K, bool SP2>
 int launch_ana(const char* name, const double2* spec, int64_t ld, int64_t smap, int nside, int Lm, const Tables& tab,

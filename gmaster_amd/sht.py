@@ -123,6 +123,7 @@ class Plan:
     nchunks: int
     tsize: int
     nchunks_mixed: int = 0
+    nslots: int = 0        # partial slots that an FP64 spin-0 pass writes
 
 
 def plan(nside, lmax, spin, device=None, polar_skip=True):
@@ -151,6 +152,7 @@ def plan(nside, lmax, spin, device=None, polar_skip=True):
         nchunks=int(_lib.query("gm_lat_nchunks", nside, spin)),
         tsize=tsize,
         nchunks_mixed=int(_lib.query("gm_lat_nchunks_mixed", nside, spin, 1)),
+        nslots=int(_lib.query("gm_lat_slots_s0", nside)),
     )
     _PLANS[key] = p
     return p
@@ -248,7 +250,7 @@ def _analysis_s0(p, spec, alm, mode, mixed=False):
     st = _lib.stream_ptr(p.device)
     nch = int(_lib.query("gm_lat_nchunks_mixed", p.nside, 0, K)) if mixed else p.nchunks
     sfx = "_mixed" if mixed else ""
-    partial = torch.empty(nch * p.tsize * 2 * K, dtype=torch.float64, device=p.device)
+    partial = torch.empty((nch if mixed else p.nslots) * p.tsize * 2 * K, dtype=torch.float64, device=p.device)
     ld = spec.shape[2]
     for c0, md in _passes(p, 0, mixed, K, nch, int(mode)):
         _lib.call("gm_lat_ana_s0" + sfx, _lib.ptr(spec), K, ld, spec.stride(0), p.nside, p.lmax, _lib.ptr(p.alpha),

@@ -105,8 +105,10 @@ int gm_lat_tables(int64_t lmax, int64_t spin, double* alpha, double* gamma, doub
 /* Spin-0 analysis of nmaps (1 or 2) phased spectra sharing one recurrence, one pass over
  * the ring chunks chunk0 .. chunk0 + nchunks - 1:
  * partial[c - chunk0][base(m) + l - m][map] = sum_{rings of chunk c} mu_lm(theta) (G_N +- G_S)
- * nchunks = gm_lat_nchunks(nside, 0) slots; chunk0 = 0, nchunks, 2 nchunks, ... below
- * gm_lat_ring_chunks (one pass up to Nside 4096; passes bound the partial buffer above).
+ * nchunks = gm_lat_nchunks(nside, 0); chunk0 = 0, nchunks, 2 nchunks, ... below
+ * gm_lat_ring_chunks (one pass up to Nside 4096; passes bound the partial buffer above).  A pass
+ * writes gm_lat_slots_s0(nside) slots at most (slots of 128 to 2048 ring pairs, whatever the
+ * chunks), which is what partial has to hold.
  * Replaces gm_march_ana_s0 / gm_march_ana_s0_pair (march_v2.cu:155-285, :551-552). */
 int gm_lat_ana_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride,
                   int64_t nside, int64_t lmax, const double* alpha, const double* seed_mant,
@@ -187,6 +189,8 @@ int gm_lat2_syn(const double* coef, const double* pcoef, int64_t nside, int64_t 
  * analysis kernels split the rings of one order into (mixed != 0: the mixed kernels with
  * nmaps maps per recurrence); passes start at chunk0 = 0, slots, 2 slots, ... */
 int64_t gm_lat_nchunks(int64_t nside, int64_t spin);
+/* Partial slots that an FP64 spin-0 analysis pass writes. */
+int64_t gm_lat_slots_s0(int64_t nside);
 int64_t gm_lat_ring_chunks(int64_t nside, int64_t spin, int64_t mixed, int64_t nmaps);
 
 /* ---------------------------------------------------------------- power spectra, MCM */
