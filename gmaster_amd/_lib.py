@@ -32,6 +32,7 @@ SIGNATURES = {
     "gm_ring_fold_residual": [_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p],
     "gm_ring_fold_residual_c": [_p, _p, _p, _i64, _i64, _i64, _p],
     "gm_lat_tables": [_i64, _i64, _p, _p, _p, _p],
+    "gm_lat_tables_orders": [_i64, _i64, _i64, _p, _p, _p, _p],
     "gm_lat_ana_s0": [_p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _p],
     "gm_lat_ana_s0_mixed": [_p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _p],
     "gm_lat_finish_s0": [_p, _i64, _i64, _p, _p, _i64, _p, _i64, _i32, _i64, _p],

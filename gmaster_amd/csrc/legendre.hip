@@ -706,10 +706,10 @@ __global__ __launch_bounds__(64 * NW) void k_syn_s_mx(const double2* __restrict_
 }
 
 // ------------------------------------------------------------------ tables
-__global__ void k_lat_tables(int L, int s, double* __restrict__ alpha, double* __restrict__ gamma,
+__global__ void k_lat_tables(int L, int s, int norders, double* __restrict__ alpha, double* __restrict__ gamma,
                              double* __restrict__ P) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= L) return;
+    if (m >= norders) return;
     const int M = m > s ? m : s;
     const int64_t base = table_base(m, L) - m;  // entry l at base + l
     const int lend = L + GM_TABLE_PAD;
@@ -999,13 +999,19 @@ extern "C" int64_t gm_lat_ring_chunks(int64_t nside, int64_t spin, int64_t mixed
     return lat_config(nside, spin, mixed != 0, (int)nmaps).nchunks;
 }
 
+extern "C" int gm_lat_tables_orders(int64_t lmax, int64_t spin, int64_t norders, double* alpha, double* gamma, double* P,
+                                    void* stream) {
+    const char* name = "gm_lat_tables";
+    if (lmax < 0 || spin < 0 || spin > lmax) return fail(GM_E_ARG, "%s: bad lmax / spin", name);
+    if (norders < 1 || norders > lmax + 1) return fail(GM_E_ARG, "%s: norders outside [1, lmax + 1]", name);
+    if (!alpha || !P || (spin && !gamma)) return fail(GM_E_ARG, "%s: null pointer", name);
+    hipLaunchKernelGGL(k_lat_tables, dim3((unsigned)((norders + 63) / 64)), dim3(64), 0, (hipStream_t)stream, (int)lmax + 1,
+                       (int)spin, (int)norders, alpha, gamma, P);
+    return check_launch(name);
+}
+
 extern "C" int gm_lat_tables(int64_t lmax, int64_t spin, double* alpha, double* gamma, double* P, void* stream) {
-    if (lmax < 0 || spin < 0 || spin > lmax) return fail(GM_E_ARG, "gm_lat_tables: bad lmax / spin");
-    if (!alpha || !P || (spin && !gamma)) return fail(GM_E_ARG, "gm_lat_tables: null pointer");
-    const int L = (int)lmax + 1;
-    hipLaunchKernelGGL(k_lat_tables, dim3((L + 63) / 64), dim3(64), 0, (hipStream_t)stream, L, (int)spin, alpha,
-                       gamma, P);
-    return check_launch("gm_lat_tables");
+    return gm_lat_tables_orders(lmax, spin, lmax + 1, alpha, gamma, P, stream);
 }
 
 

@@ -135,16 +135,23 @@ def plan(nside, lmax, spin, device=None, polar_skip=True):
     p = _PLANS.get(key)
     if p is not None:
         return p
-    nside, lmax, spin = int(nside), int(lmax), int(spin)
+    p = _make_plan(int(nside), int(lmax), int(spin), device, polar_skip, int(lmax) + 1)
+    _PLANS[key] = p
+    return p
+
+
+def _make_plan(nside, lmax, spin, device, polar_skip, norders):
+    """Tables of the orders m < norders (the head of the full tables)."""
     L = lmax + 1
-    tsize = int(_lib.query("gm_table_size", lmax))
+    tsize = norders * (L + 8) - norders * (norders - 1) // 2
     f64 = dict(dtype=torch.float64, device=device)
     alpha = torch.empty(tsize, **f64)
     gamma = torch.empty(tsize, **f64) if spin else None
     P = torch.empty(tsize, **f64)
-    _lib.call("gm_lat_tables", lmax, spin, _lib.ptr(alpha), _lib.ptr(gamma), _lib.ptr(P), _lib.stream_ptr(device))
+    _lib.call("gm_lat_tables_orders", lmax, spin, norders, _lib.ptr(alpha), _lib.ptr(gamma), _lib.ptr(P),
+              _lib.stream_ptr(device))
     sm, se = _seed_constants(L, spin)
-    p = Plan(
+    return Plan(
         nside=nside, lmax=lmax, spin=spin, device=device, alpha=alpha, gamma=gamma, P=P,
         smant=torch.as_tensor(sm, **f64),
         sexp=torch.as_tensor(se, dtype=torch.int32, device=device),
@@ -154,8 +161,6 @@ def plan(nside, lmax, spin, device=None, polar_skip=True):
         nchunks_mixed=int(_lib.query("gm_lat_nchunks_mixed", nside, spin, 1)),
         nslots=int(_lib.query("gm_lat_slots_s0", nside)),
     )
-    _PLANS[key] = p
-    return p
 
 
 # Ring pairs with sin^2(theta) below this run the spin-2 recurrence itself; the others the
@@ -175,7 +180,7 @@ class Plan2:
     lmax: int
     device: torch.device
     tab: Plan              # spin-0 tables of lmax + 2
-    pol: Plan              # spin-2 tables (polar rings)
+    pol: Plan              # spin-2 tables of the orders m < mpol (polar rings)
     nact: torch.Tensor     # ring pairs visited by order m
     jsplit: int            # first ring pair of the polar part
     mpol: int              # orders that reach the polar rings, LOW_ORDERS at least
@@ -201,7 +206,7 @@ def plan2(nside, lmax, device=None, polar_skip=True):
     mpol = max(mpol, min(LOW_ORDERS, L))
     p = Plan2(
         nside=nside, lmax=lmax, device=device, tab=plan(nside, lmax + 2, 0, device, polar_skip),
-        pol=plan(nside, lmax, 2, device, polar_skip),
+        pol=_make_plan(nside, lmax, 2, device, polar_skip, mpol),
         nact=torch.as_tensor(_nactive_pairs(nside, lmax, polar_skip), dtype=torch.int32, device=device),
         jsplit=jsplit, mpol=mpol, nslots=int(_lib.query("gm_lat2_slots", nside, jsplit)),
         nchunks=int(_lib.query("gm_lat2_chunks", nside, jsplit)),

@@ -101,6 +101,10 @@ int gm_ring_fold_residual_c(const double* F, const double* G, double* R, int64_t
  * seed_mant / seed_exp (lmax+1 entries, host-computed) are passed to the kernels below.
  * Replaces the window tables of gmaster/_sht/march_v2.py:388-450. */
 int gm_lat_tables(int64_t lmax, int64_t spin, double* alpha, double* gamma, double* P, void* stream);
+/* The orders m < norders alone, the head of the full tables: norders (lmax + 9) -
+ * norders (norders - 1) / 2 doubles each. */
+int gm_lat_tables_orders(int64_t lmax, int64_t spin, int64_t norders, double* alpha, double* gamma, double* P,
+                         void* stream);
 
 /* Spin-0 analysis of nmaps (1 or 2) phased spectra sharing one recurrence, one pass over
  * the ring chunks chunk0 .. chunk0 + nchunks - 1:

@@ -24,3 +24,22 @@ def test_spin0_partial_sums(nside, maps):
     used = torch.cuda.memory_stats()["requested_bytes.all.peak"] - base
     slots = {64: 1, 512: 2, 1024: 1, 2048: 2}[nside]
     assert used <= slots * int(_lib.query("gm_table_size", lmax)) * 16 * maps
+
+
+@pytest.mark.parametrize("nside,lmax", [(256, 767), (512, 1535)])
+def test_spin2_tables(nside, lmax):
+    """The spin-2 tables that a geometry keeps beside the spin-0 ones: the orders of the polar rings
+    alone, equal to the head of the full tables."""
+    from gmaster_amd import _lib, sht
+
+    sht.clear_plans()
+    dev = torch.device("cuda", torch.cuda.current_device())
+    base = torch.cuda.memory_stats()["requested_bytes.all.current"]
+    p = sht.plan2(nside, lmax, dev)
+    kept = torch.cuda.memory_stats()["requested_bytes.all.current"] - base
+    assert p.mpol < (lmax + 1) // 3
+    tables = 2 * int(_lib.query("gm_table_size", lmax + 2)) + 3 * p.ptsize
+    assert kept <= 8 * tables + 64 * (lmax + 3)  # and a few numbers per order
+    full = sht.plan(nside, lmax, 2, dev)
+    for name in ("alpha", "gamma", "P"):
+        assert torch.equal(getattr(p.pol, name), getattr(full, name)[:p.ptsize])
