@@ -63,10 +63,9 @@ __device__ inline void block_reduce(const F (&acc)[NV], F* lds, int buf, double*
 
 // ------------------------------------------------------------------ spin-0 analysis
 // Folded lanes: j = 0 is the equator ring, j > 0 the pair (north r = 2n-1-j, south 2n-1+j).
-// The recurrence always runs in FP64; F is the arithmetic type of the contraction: each
-// step's mu is rounded to F once and multiplied into F accumulators (spectra are read as
-// FP64 and converted, partial sums stored in FP64).
-template <int K, int R, int NW, typename F>
+// The recurrence runs in FP64; each step's mu is rounded to FP32 once and multiplied into FP32
+// accumulators (spectra are read as FP64 and converted, partial sums stored in FP64).
+template <int K, int R, int NW>
 __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ spec, int64_t ld,
                                                     int64_t smap, int nside, int L,
                                                     const double* __restrict__ alpha,
@@ -77,7 +76,7 @@ __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ 
     constexpr int NV = 4 * 2 * K;  // 4 degrees x (re, im) x maps
     constexpr int T = 64 * NW;
     constexpr int CH = T * R;
-    __shared__ F lds[2 * NV * T];
+    __shared__ float lds[2 * NV * T];
     // ring chunk chunk0 + blockIdx.x, written to partial slot blockIdx.x
     const int c = chunk0 + blockIdx.x, m = blockIdx.y;
     const int na = nact[m];
@@ -85,7 +84,7 @@ __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ 
 
     double x[R], mu0[R], mu1[R];
     int kx[R];
-    cpx<F> gE[R][K], gO[R][K];
+    cpx<float> gE[R][K], gO[R][K];
     const double sm = smant[m];
     const int se = sexp[m];
 #pragma unroll
@@ -101,12 +100,12 @@ __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ 
             for (int k = 0; k < K; ++k) {
                 const double2 a = spec[k * smap + (int64_t)r * ld + m];
                 if (j == 0) {
-                    gE[t][k] = cpx<F>{(F)a.x, (F)a.y};
-                    gO[t][k] = cpx<F>{0, 0};
+                    gE[t][k] = cpx<float>{(float)a.x, (float)a.y};
+                    gO[t][k] = cpx<float>{0, 0};
                 } else {
                     const double2 b = spec[k * smap + (int64_t)rp * ld + m];
-                    gE[t][k] = cpx<F>{(F)(a.x + b.x), (F)(a.y + b.y)};
-                    gO[t][k] = cpx<F>{(F)(a.x - b.x), (F)(a.y - b.y)};
+                    gE[t][k] = cpx<float>{(float)(a.x + b.x), (float)(a.y + b.y)};
+                    gO[t][k] = cpx<float>{(float)(a.x - b.x), (float)(a.y - b.y)};
                 }
             }
         } else {
@@ -114,7 +113,7 @@ __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ 
             mu0[t] = 0;
             kx[t] = 0;
 #pragma unroll
-            for (int k = 0; k < K; ++k) gE[t][k] = gO[t][k] = cpx<F>{0, 0};
+            for (int k = 0; k < K; ++k) gE[t][k] = gO[t][k] = cpx<float>{0, 0};
         }
     }
     bool anyinact = false;
@@ -137,7 +136,7 @@ __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ 
             a[i] = an[i];
             an[i] = al[l0 + 4 + i + 1];  // prefetch the next block's coefficients
         }
-        F acc[NV];
+        float acc[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) acc[v] = 0;
 #pragma unroll
@@ -145,10 +144,10 @@ __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ 
             // l0 + m is even, so degree l0 + i pairs with the even (E) combination for even i
 #pragma unroll
             for (int t = 0; t < R; ++t) {
-                const F cur = (F)((i & 1) ? mu1[t] : mu0[t]);
+                const float cur = (float)((i & 1) ? mu1[t] : mu0[t]);
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
-                    const cpx<F> gv = (i & 1) ? gO[t][k] : gE[t][k];
+                    const cpx<float> gv = (i & 1) ? gO[t][k] : gE[t][k];
                     acc[i * 2 * K + 2 * k] = fma(cur, gv.x, acc[i * 2 * K + 2 * k]);
                     acc[i * 2 * K + 2 * k + 1] = fma(cur, gv.y, acc[i * 2 * K + 2 * k + 1]);
                 }
@@ -160,119 +159,7 @@ __global__ __launch_bounds__(64 * NW) void k_ana_s0(const double2* __restrict__ 
             }
         }
         rescale<R, double>(mu0, mu1, kx, anyinact);
-        block_reduce<NV, NW, F>(acc, lds, buf, part + (int64_t)l0 * (2 * K));
-    }
-}
-
-// ------------------------------------------------------------------ spin-0 synthesis
-template <int K, int R, int NW, typename F>
-__global__ __launch_bounds__(64 * NW) void k_syn_s0(const double2* __restrict__ coef, int nside, int L,
-                                                    const double* __restrict__ alpha,
-                                                    const double* __restrict__ smant,
-                                                    const int* __restrict__ sexp,
-                                                    const int* __restrict__ nact,
-                                                    double2* __restrict__ spec, int64_t ld, int64_t smap) {
-    constexpr int T = 64 * NW;
-    constexpr int CH = T * R;
-    const int c = blockIdx.x, m = blockIdx.y;
-    const int na = nact[m];
-    const int NF = 2 * nside;
-
-    double x[R], mu0[R], mu1[R];
-    int kx[R];
-    cpx<F> aE[R][K], aO[R][K];
-    const double sm = smant[m];
-    const int se = sexp[m];
-    bool anyact = false;
-#pragma unroll
-    for (int t = 0; t < R; ++t) {
-        const int j = c * CH + t * T + threadIdx.x;
-        mu1[t] = 0;
-        kx[t] = 0;
-        x[t] = 0;
-        mu0[t] = 0;
-        if (j < na) {
-            const Ring g = ring_info(nside, 2 * nside - 1 - j);
-            x[t] = g.z;
-            seed_lane<double>(sm, se, m, m, g.shalf, g.chalf, mu0[t], kx[t]);
-            anyact = true;
-        }
-#pragma unroll
-        for (int k = 0; k < K; ++k) aE[t][k] = aO[t][k] = cpx<F>{0, 0};
-    }
-    if (__any(anyact)) {
-        bool anyinact = false;
-#pragma unroll
-        for (int t = 0; t < R; ++t) anyinact = anyinact || (kx[t] < 0);
-        anyinact = __any(anyinact);
-        const double* al = alpha + table_base(m, L) - m;
-        const double2* cf = coef + (table_base(m, L) - m) * K;
-        double an[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) an[i] = al[m + i + 1];
-        // one or two maps: the next block's coefficients are prefetched; for batches the
-        // 4K uniform values would not fit the scalar registers twice, so they load in place
-        constexpr int KP = K <= 2 ? K : 1;
-        cpx<F> cn[4][KP];
-        if constexpr (K <= 2) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < K; ++k) cn[i][k] = load_c<F>(cf + (int64_t)(m + i) * K + k);
-        }
-        for (int l0 = m; l0 < L; l0 += 4) {
-            double a[4];
-            cpx<F> cb[4][K];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = an[i];
-                an[i] = al[l0 + 4 + i + 1];
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    if constexpr (K <= 2) {
-                        cb[i][k] = cn[i][k];
-                        cn[i][k] = load_c<F>(cf + (int64_t)(l0 + 4 + i) * K + k);  // next block (zero padded)
-                    } else {
-                        cb[i][k] = load_c<F>(cf + (int64_t)(l0 + i) * K + k);
-                    }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                cpx<F> cv[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k) cv[k] = cb[i][k];
-#pragma unroll
-                for (int t = 0; t < R; ++t) {
-                    const F cur = (F)((i & 1) ? mu1[t] : mu0[t]);
-#pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        cpx<F>& acc = (i & 1) ? aO[t][k] : aE[t][k];
-                        acc.x = fma(cur, cv[k].x, acc.x);
-                        acc.y = fma(cur, cv[k].y, acc.y);
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < R; ++t) {
-                    if (i & 1) mu0[t] = fma(x[t] * a[i], mu1[t], -mu0[t]);
-                    else mu1[t] = fma(x[t] * a[i], mu0[t], -mu1[t]);
-                }
-            }
-            rescale<R, double>(mu0, mu1, kx, anyinact);
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < R; ++t) {
-        const int j = c * CH + t * T + threadIdx.x;
-        if (j >= NF) continue;
-        const int r = 2 * nside - 1 - j, rp = 2 * nside - 1 + j;
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            // F_N = E + O, F_S = E - O (zero for rings beyond the polar-skip bound)
-            const double ex = aE[t][k].x, ey = aE[t][k].y, ox = aO[t][k].x, oy = aO[t][k].y;
-            spec[k * smap + (int64_t)r * ld + m] = make_double2(ex + ox, ey + oy);
-            if (j > 0) spec[k * smap + (int64_t)rp * ld + m] = make_double2(ex - ox, ey - oy);
-        }
+        block_reduce<NV, NW, float>(acc, lds, buf, part + (int64_t)l0 * (2 * K));
     }
 }
 
@@ -864,9 +751,9 @@ __global__ void k_prep_s(const double2* __restrict__ ae, const double2* __restri
 // ------------------------------------------------------------------ configs
 // Large geometries use 4-wave workgroups with R rings per lane, per precision and pass
 // (the mixed kernels hold half the registers per ring; the mixed syntheses keep their
-// accumulators in MFMA tiles).  The FP64 spin-0 kernels (pairs.hip) have shapes of their own;
-// here the FP64 spin-0 analysis only has its pass and slot counts.  Chosen by timing R = 3..10 on MI355X at Nside 4096:
-// occupancy steps make the best R differ between passes.
+// accumulators in MFMA tiles).  Chosen by timing R = 3..10 on MI355X at Nside 4096: occupancy steps
+// make the best R differ between passes.  The FP64 spin-0 kernels (pairs.hip) have shapes of
+// their own; here GM_ANA_R_S0 counts the chunks of their passes.
 #ifndef GM_ANA_R_S0
 #define GM_ANA_R_S0 6
 #endif
@@ -1052,7 +939,7 @@ int launch_ana_s0_mixed(const char* name, const double* spec, int64_t nmaps, int
     const double2* sp = reinterpret_cast<const double2*>(spec);
     constexpr int RL = large_r(false, true, true);
     if (int e = check_config(name, cfg, large_r(false, true, true, (int)nmaps))) return e;
-#define GM_ANA0(KK, RR, WW) hipLaunchKernelGGL((k_ana_s0<KK, RR, WW, float>), grid, block, 0, st, sp, ld, smap, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, partial, ts, (int)chunk0)
+#define GM_ANA0(KK, RR, WW) hipLaunchKernelGGL((k_ana_s0<KK, RR, WW>), grid, block, 0, st, sp, ld, smap, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, partial, ts, (int)chunk0)
     if (nmaps == 1) {
         if (cfg.NW == 1) GM_ANA0(1, 2, 1);
         else if (cfg.NW == 2) GM_ANA0(1, 4, 2);
@@ -1074,12 +961,6 @@ int launch_ana_s0_mixed(const char* name, const double* spec, int64_t nmaps, int
     return check_launch(name);
 }
 
-// A single mixed spin-0 map (K = 1) synthesises on the matrix unit when this is 1, else on
-// the vector ALU in FP32.
-#ifndef GM_MIX_SYN0_SINGLE_MFMA
-#define GM_MIX_SYN0_SINGLE_MFMA 1
-#endif
-
 int launch_syn_s0_mixed(const char* name, const double* coef, int64_t nmaps, int64_t nside, int64_t lmax,
                         const double* alpha, const double* seed_mant, const int32_t* seed_exp, const int32_t* nactive,
                         double* spec, int64_t ld, int64_t smap, void* stream) {
@@ -1093,15 +974,7 @@ int launch_syn_s0_mixed(const char* name, const double* coef, int64_t nmaps, int
     double2* sp = reinterpret_cast<double2*>(spec);
     constexpr int RL = large_r(true, true, true);
     if (int e = check_config(name, cfg, large_r(true, true, true, (int)nmaps))) return e;
-#define GM_SYN0(KK, RR, WW)                                                                                       \
-    do {                                                                                                          \
-        if constexpr (KK > 1 || GM_MIX_SYN0_SINGLE_MFMA)                                                          \
-            hipLaunchKernelGGL((k_syn_s0_mx<KK, RR, WW>), grid, block, 0, st, cf, (int)nside, (int)L, alpha,      \
-                               seed_mant, seed_exp, nactive, sp, ld, smap);                                        \
-        else                                                                                                      \
-            hipLaunchKernelGGL((k_syn_s0<KK, RR, WW, float>), grid, block, 0, st, cf, (int)nside, (int)L, alpha,  \
-                               seed_mant, seed_exp, nactive, sp, ld, smap);                                        \
-    } while (0)
+#define GM_SYN0(KK, RR, WW) hipLaunchKernelGGL((k_syn_s0_mx<KK, RR, WW>), grid, block, 0, st, cf, (int)nside, (int)L, alpha, seed_mant, seed_exp, nactive, sp, ld, smap)
     if (nmaps == 1) {
         if (cfg.NW == 1) GM_SYN0(1, 2, 1);
         else if (cfg.NW == 2) GM_SYN0(1, 4, 2);
