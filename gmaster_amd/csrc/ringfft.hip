@@ -1153,15 +1153,15 @@ using namespace gm;
 
 namespace {
 
-int ring_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside, int64_t lmax, double* spec,
-                int64_t ld, int64_t spec_map_stride, void* stream, bool pairs) {
+int ring_fwd_s0(const char* name, const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside, int64_t lmax,
+                double* spec, int64_t ld, int64_t spec_map_stride, void* stream, bool pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
-    if (!maps || !spec) return fail(GM_E_ARG, "gm_ring_fft_fwd_s0: null pointer");
+    if (!maps || !spec) return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t L = lmax + 1, npix = 12 * nside * nside, nring = 4 * nside - 1;
-    if (nmaps < 1) return fail(GM_E_ARG, "gm_ring_fft_fwd_s0: nmaps must be >= 1");
-    if (ld < L) return fail(GM_E_SHAPE, "gm_ring_fft_fwd_s0: ld (%lld) < lmax + 1", (long long)ld);
+    if (nmaps < 1) return fail(GM_E_ARG, "%s: nmaps must be >= 1", name);
+    if (ld < L) return fail(GM_E_SHAPE, "%s: ld (%lld) < lmax + 1", name, (long long)ld);
     if (nmaps > 1 && (map_stride < npix || spec_map_stride < nring * ld))
-        return fail(GM_E_SHAPE, "gm_ring_fft_fwd_s0: map strides too small");
+        return fail(GM_E_SHAPE, "%s: map strides too small", name);
     if (pairs) {
         const RingArgs ra{maps, nullptr, map_stride, (int)nmaps, (int)nside, (int)L, reinterpret_cast<double2*>(spec),
                           ld, spec_map_stride, (hipStream_t)stream};
@@ -1192,15 +1192,15 @@ int ring_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t n
                                (int)L, b[i].qlo, b[i].qhi, sp, ld, spec_map_stride, dcap);
         }
     }
-    return check_launch("gm_ring_fft_fwd_s0");
+    return check_launch(name);
 }
 
-int ring_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec, int64_t ld, void* stream,
-               bool pairs) {
+int ring_fwd_s(const char* name, const double* q, const double* u, int64_t nside, int64_t lmax, double* spec, int64_t ld,
+               void* stream, bool pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
-    if (!q || !u || !spec) return fail(GM_E_ARG, "gm_ring_fft_fwd_s: null pointer");
+    if (!q || !u || !spec) return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t L = lmax + 1;
-    if (ld < 2 * L - 1) return fail(GM_E_SHAPE, "gm_ring_fft_fwd_s: ld (%lld) < 2 lmax + 1", (long long)ld);
+    if (ld < 2 * L - 1) return fail(GM_E_SHAPE, "%s: ld (%lld) < 2 lmax + 1", name, (long long)ld);
     if (pairs) {
         const RingArgs ra{q, u, 0, 1, (int)nside, (int)L, reinterpret_cast<double2*>(spec), ld, 0,
                           (hipStream_t)stream};
@@ -1231,18 +1231,18 @@ int ring_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, do
                                b[i].qlo, b[i].qhi, sp, ld, dcap);
         }
     }
-    return check_launch("gm_ring_fft_fwd_s");
+    return check_launch(name);
 }
 
-int ring_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride, int64_t nside, int64_t lmax,
-                double* maps, int64_t map_stride, void* stream, bool pairs) {
+int ring_inv_s0(const char* name, const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride, int64_t nside,
+                int64_t lmax, double* maps, int64_t map_stride, void* stream, bool pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
-    if (!maps || !spec) return fail(GM_E_ARG, "gm_ring_fft_inv_s0: null pointer");
+    if (!maps || !spec) return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t L = lmax + 1, npix = 12 * nside * nside, nring = 4 * nside - 1;
-    if (nmaps < 1) return fail(GM_E_ARG, "gm_ring_fft_inv_s0: nmaps must be >= 1");
-    if (ld < L) return fail(GM_E_SHAPE, "gm_ring_fft_inv_s0: ld < lmax + 1");
+    if (nmaps < 1) return fail(GM_E_ARG, "%s: nmaps must be >= 1", name);
+    if (ld < L) return fail(GM_E_SHAPE, "%s: ld < lmax + 1", name);
     if (nmaps > 1 && (map_stride < npix || spec_map_stride < nring * ld))
-        return fail(GM_E_SHAPE, "gm_ring_fft_inv_s0: map strides too small");
+        return fail(GM_E_SHAPE, "%s: map strides too small", name);
     if (pairs) {
         const RingArgs ra{maps, nullptr, map_stride, (int)nmaps, (int)nside, (int)L,
                           reinterpret_cast<double2*>(const_cast<double*>(spec)), ld, spec_map_stride,
@@ -1274,15 +1274,15 @@ int ring_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_
                                (int)nside, (int)L, b[i].qlo, b[i].qhi, maps, map_stride, dcap);
         }
     }
-    return check_launch("gm_ring_fft_inv_s0");
+    return check_launch(name);
 }
 
-int ring_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q, double* u, void* stream, bool
-               pairs) {
+int ring_inv_s(const char* name, const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q, double* u,
+               void* stream, bool pairs) {
     if (int e = check_ring_args(nside, lmax)) return e;
-    if (!spec || !q || !u) return fail(GM_E_ARG, "gm_ring_fft_inv_s: null pointer");
+    if (!spec || !q || !u) return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t L = lmax + 1;
-    if (ld < 2 * L - 1) return fail(GM_E_SHAPE, "gm_ring_fft_inv_s: ld < 2 lmax + 1");
+    if (ld < 2 * L - 1) return fail(GM_E_SHAPE, "%s: ld < 2 lmax + 1", name);
     if (pairs) {
         const RingArgs ra{q, u, 0, 1, (int)nside, (int)L, reinterpret_cast<double2*>(const_cast<double*>(spec)), ld,
                           0, (hipStream_t)stream};
@@ -1313,49 +1313,49 @@ int ring_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, doub
                                b[i].qlo, b[i].qhi, q, u, dcap);
         }
     }
-    return check_launch("gm_ring_fft_inv_s");
+    return check_launch(name);
 }
 
 }  // namespace
 
 extern "C" int gm_ring_fft_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside, int64_t lmax,
                                   double* spec, int64_t ld, int64_t spec_map_stride, void* stream) {
-    return ring_fwd_s0(maps, nmaps, map_stride, nside, lmax, spec, ld, spec_map_stride, stream, false);
+    return ring_fwd_s0("gm_ring_fft_fwd_s0", maps, nmaps, map_stride, nside, lmax, spec, ld, spec_map_stride, stream, false);
 }
 
 extern "C" int gm_ring_pair_fwd_s0(const double* maps, int64_t nmaps, int64_t map_stride, int64_t nside, int64_t lmax,
                                    double* spec, int64_t ld, int64_t spec_map_stride, void* stream) {
-    return ring_fwd_s0(maps, nmaps, map_stride, nside, lmax, spec, ld, spec_map_stride, stream, true);
+    return ring_fwd_s0("gm_ring_pair_fwd_s0", maps, nmaps, map_stride, nside, lmax, spec, ld, spec_map_stride, stream, true);
 }
 
 extern "C" int gm_ring_fft_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec, int64_t
                                  ld, void* stream) {
-    return ring_fwd_s(q, u, nside, lmax, spec, ld, stream, false);
+    return ring_fwd_s("gm_ring_fft_fwd_s", q, u, nside, lmax, spec, ld, stream, false);
 }
 
 extern "C" int gm_ring_pair_fwd_s(const double* q, const double* u, int64_t nside, int64_t lmax, double* spec, int64_t
                                   ld, void* stream) {
-    return ring_fwd_s(q, u, nside, lmax, spec, ld, stream, true);
+    return ring_fwd_s("gm_ring_pair_fwd_s", q, u, nside, lmax, spec, ld, stream, true);
 }
 
 extern "C" int gm_ring_fft_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride, int64_t
                                   nside, int64_t lmax, double* maps, int64_t map_stride, void* stream) {
-    return ring_inv_s0(spec, nmaps, ld, spec_map_stride, nside, lmax, maps, map_stride, stream, false);
+    return ring_inv_s0("gm_ring_fft_inv_s0", spec, nmaps, ld, spec_map_stride, nside, lmax, maps, map_stride, stream, false);
 }
 
 extern "C" int gm_ring_pair_inv_s0(const double* spec, int64_t nmaps, int64_t ld, int64_t spec_map_stride, int64_t
                                    nside, int64_t lmax, double* maps, int64_t map_stride, void* stream) {
-    return ring_inv_s0(spec, nmaps, ld, spec_map_stride, nside, lmax, maps, map_stride, stream, true);
+    return ring_inv_s0("gm_ring_pair_inv_s0", spec, nmaps, ld, spec_map_stride, nside, lmax, maps, map_stride, stream, true);
 }
 
 extern "C" int gm_ring_fft_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q, double* u,
                                  void* stream) {
-    return ring_inv_s(spec, ld, nside, lmax, q, u, stream, false);
+    return ring_inv_s("gm_ring_fft_inv_s", spec, ld, nside, lmax, q, u, stream, false);
 }
 
 extern "C" int gm_ring_pair_inv_s(const double* spec, int64_t ld, int64_t nside, int64_t lmax, double* q, double* u,
                                   void* stream) {
-    return ring_inv_s(spec, ld, nside, lmax, q, u, stream, true);
+    return ring_inv_s("gm_ring_pair_inv_s", spec, ld, nside, lmax, q, u, stream, true);
 }
 
 extern "C" int gm_ring_fold_residual(const double* F, const double* G, double* R, int64_t nmaps, int64_t ld,
