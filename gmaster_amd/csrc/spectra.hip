@@ -86,8 +86,8 @@ __global__ void k_bin_cell(const double* __restrict__ cl, int64_t ld, const int*
 // the rows of b1 (eight rows in flight), then the columns' products meet in LDS and one thread
 // per bin adds its own, 256 columns at a time.  Bound: HBM for wide matrices, else latency.  One
 // thread per bin read a cache line per column (16 degrees a bin: ten times the matrix's bytes,
-// 2.7 ms a block at lmax 12287 -> 0.21) and one row after the other (115 us for a
-// 3072 x 3072 block, 4 degrees a bin -> 19 us).  All blocks and slots are one launch: eight slots
+// 1.7 ms a block at lmax 12287 -> 0.21) and one row after the other (26 us for a 3000 x 3000
+// block, 4 degrees a bin -> 16; 106 -> 16 with 16 a bin).  All blocks and slots are one launch: eight slots
 // of two blocks were 2 + 16 launches.
 constexpr int kBinSlots = 16;  // of one launch
 template <int N> struct Rows { static constexpr int value = N; };
@@ -98,51 +98,71 @@ struct BinBlocks {
     signed char block[kBinSlots], c1[kBinSlots], c2[kBinSlots], sign[kBinSlots];
 };
 
+// NB1 bins b1 per workgroup (blockIdx.y): their rows' loads, LDS words and barriers run together.
+template <int NB1>
 __global__ __launch_bounds__(256) void k_bin_blocks(BinBlocks bb, int L, const int* __restrict__ ells,
                                                     const int* __restrict__ bstart, int nb,
                                                     const double* __restrict__ wout, const double* __restrict__ tin,
                                                     int ncls, int nbw, double* __restrict__ out) {
-    __shared__ double val[256];
+    __shared__ double val[NB1][256];
     const int tid = threadIdx.x;
-    const int b1 = blockIdx.y, z = blockIdx.z;
+    const int b10 = blockIdx.y * NB1, z = blockIdx.z;
     const int first = blockIdx.x * nbw, b2 = first + tid;
     const bool mine = tid < nbw && b2 < nb;
     const double* __restrict__ M = bb.M[z];
     const int lo = mine ? bstart[b2] : 0, hi = mine ? bstart[b2 + 1] : 0;
     const int c_end = bstart[min(first + nbw, nb)];
-    const int r0 = bstart[b1], end = bstart[b1 + 1];
-    double s = 0.0;
+    int row[NB1 + 1];  // bins past the last are empty
+#pragma unroll
+    for (int q = 0; q <= NB1; ++q) row[q] = bstart[min(b10 + q, nb)];
+    double s[NB1];
+#pragma unroll
+    for (int q = 0; q < NB1; ++q) s[q] = 0.0;
     for (int c0 = bstart[first]; c0 < c_end; c0 += 256) {
         const int e2 = c0 + tid;
-        double v = 0.0;
+        double v[NB1];
+#pragma unroll
+        for (int q = 0; q < NB1; ++q) v[q] = 0.0;
         if (e2 < c_end) {
             const int c = ells[e2];
-            auto rows = [&](auto n, int e1) {
-                double m[n.value];
 #pragma unroll
-                for (int u = 0; u < n.value; ++u) m[u] = M[(int64_t)ells[e1 + u] * L + c];
+            for (int q = 0; q < NB1; ++q) {
+                auto rows = [&](auto n, int e1) {
+                    double m[n.value];
 #pragma unroll
-                for (int u = 0; u < n.value; ++u) v = fma(wout[e1 + u], m[u], v);
-            };
-            int e1 = r0;
-            for (; e1 + 8 <= end; e1 += 8) rows(Rows<8>{}, e1);
-            if (e1 + 4 <= end) {
-                rows(Rows<4>{}, e1);
-                e1 += 4;
+                    for (int u = 0; u < n.value; ++u) m[u] = M[(int64_t)ells[e1 + u] * L + c];
+#pragma unroll
+                    for (int u = 0; u < n.value; ++u) v[q] = fma(wout[e1 + u], m[u], v[q]);
+                };
+                const int end = row[q + 1];
+                int e1 = row[q];
+                for (; e1 + 8 <= end; e1 += 8) rows(Rows<8>{}, e1);
+                if (e1 + 4 <= end) {
+                    rows(Rows<4>{}, e1);
+                    e1 += 4;
+                }
+                for (; e1 < end; ++e1) rows(Rows<1>{}, e1);
             }
-            for (; e1 < end; ++e1) rows(Rows<1>{}, e1);
-            v *= tin[e2];
+            const double t = tin[e2];
+#pragma unroll
+            for (int q = 0; q < NB1; ++q) v[q] *= t;
         }
-        val[tid] = v;
+#pragma unroll
+        for (int q = 0; q < NB1; ++q) val[q][tid] = v[q];
         __syncthreads();
-        for (int e = max(lo, c0); e < min(hi, c0 + 256); ++e) s += val[e - c0];
+        for (int e = max(lo, c0); e < min(hi, c0 + 256); ++e)
+#pragma unroll
+            for (int q = 0; q < NB1; ++q) s[q] += val[q][e - c0];
         __syncthreads();
     }
     if (!mine) return;
     for (int k = 0; k < bb.nslots; ++k)
         if (bb.block[k] == z)
-            out[((int64_t)b1 * ncls + bb.c1[k]) * ((int64_t)nb * ncls) + (int64_t)b2 * ncls + bb.c2[k]] =
-                bb.sign[k] < 0 ? -s : s;
+#pragma unroll
+            for (int q = 0; q < NB1; ++q)
+                if (b10 + q < nb)
+                    out[((int64_t)(b10 + q) * ncls + bb.c1[k]) * ((int64_t)nb * ncls) + (int64_t)b2 * ncls + bb.c2[k]] =
+                        bb.sign[k] < 0 ? -s[q] : s[q];
 }
 
 }  // namespace
@@ -251,9 +271,14 @@ extern "C" int gm_bin_blocks(const double* const* blocks, int64_t nblocks, int64
         if (v[0] < 0 || v[0] >= nblocks || v[1] < 0 || v[1] >= ncls || v[2] < 0 || v[2] >= ncls || (v[3] != 1 && v[3] != -1))
             return fail(GM_E_ARG, "gm_bin_blocks: bad slot %lld", (long long)k);
     }
-    // 256 columns a workgroup: 64 bins of four degrees or more, 256 narrower ones (lmax 3071, bins of
-    // one degree: 128 us in 64s, 46 in 256s)
-    const int nbw = 3 * nbands > lmax + 1 ? 256 : 64;
+    // 256 columns a workgroup: 64 bins of three degrees or more, 256 narrower ones (lmax 3071, bins of
+    // one degree: 128 us in 64s, 46 in 256s).  Bins below 3.5 degrees whose workgroups of one bin b1
+    // would fill the chip more than once (8 of them a CU) go two b1 to a workgroup, which is all
+    // latency: lmax 3000, 1 / 2 / 3 degrees a bin 42 / 23 / 23 us with one, 33 / 22 / 16 with
+    // two, 31 / 23 / 20 with four (6000: 215 / 108 / 114, 181 / 91 / 78, 155 / 90 / 73); fewer
+    // workgroups are slower in pairs (lmax 1000, 3 a bin: 4.5 us in 64s, 6.8).
+    const bool pairs = 7 * nbands > 2 * (lmax + 1) && nbands * ((nbands + 255) / 256) > 2048;
+    const int nbw = pairs || 3 * nbands > lmax + 1 ? 256 : 64, nb1 = pairs ? 2 : 1;
     // kBinSlots slots a launch: every layout of the workspaces but one block per channel pair of a
     // joint TEB workspace (49) is one launch
     for (int64_t k0 = 0; k0 < nslots; k0 += kBinSlots) {
@@ -270,7 +295,8 @@ extern "C" int gm_bin_blocks(const double* const* blocks, int64_t nblocks, int64
             bb.c2[k] = (signed char)v[2];
             bb.sign[k] = (signed char)v[3];
         }
-        hipLaunchKernelGGL(k_bin_blocks, dim3((unsigned)((nbands + nbw - 1) / nbw), (unsigned)nbands, (unsigned)used),
+        hipLaunchKernelGGL(pairs ? &k_bin_blocks<2> : &k_bin_blocks<1>,
+                           dim3((unsigned)((nbands + nbw - 1) / nbw), (unsigned)((nbands + nb1 - 1) / nb1), (unsigned)used),
                            dim3(256), 0, (hipStream_t)stream, bb, (int)(lmax + 1), ells, band_start, (int)nbands, wout, tin,
                            (int)ncls, nbw, out);
     }

@@ -1,5 +1,5 @@
 """gm_bin_block beyond one tile: more than 256 columns and more than 64 or 256 bins (both bin counts
-of a workgroup), bins across the 256-column boundary, a last partial group of bins, uneven bands with
+of a workgroup, one and two rows of bins), bins across the 256-column boundary, a last partial group of bins, uneven bands with
 gaps.  Tolerance: n + 4 roundings of the largest term for a sum of n terms."""
 
 import numpy as np
@@ -25,7 +25,7 @@ def _bands(kind, lmax):
     return ells, start
 
 
-@pytest.mark.parametrize("kind,lmax", [(1, 600), (1, 257), (2, 900), (3, 1000), (7, 999), (100, 700), (300, 900),
+@pytest.mark.parametrize("kind,lmax", [(1, 600), (1, 257), (1, 768), (2, 900), (2, 2100), (3, 1000), (3, 2200), (7, 999), (100, 700), (300, 900),
                                        ("uneven", 1000)])
 def test_bin_block_tiles(kind, lmax):
     from gmaster_amd import _lib
