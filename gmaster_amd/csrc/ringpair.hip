@@ -39,6 +39,12 @@ __device__ inline double2 cis_pi(int num, int den, double sgn) {  // e^{sgn i pi
     return make_double2(c, s);
 }
 
+__device__ inline double2 cis_minus(double x) {  // e^{-i pi x}
+    double s, c;
+    sincospi(x, &s, &c);
+    return make_double2(c, -s);
+}
+
 template <bool INV>
 __device__ __forceinline__ double2 mul_i(double2 a) {  // times -i (forward) or i (inverse)
     return INV ? make_double2(-a.y, a.x) : make_double2(a.y, -a.x);
@@ -108,9 +114,8 @@ __device__ __forceinline__ void dft(double2* v) {
     }
 }
 
-// v[j] *= w^j (j < 16), w^j as w^{4 a} w^b.
-__device__ __forceinline__ void twiddle16(double2 (&v)[16], double2 w) {
-    const double2 w2 = cmul(w, w), w3 = cmul(w2, w), w4 = cmul(w2, w2);
+// v[j] *= w^j (j < 16), w^j as w4^a w^b.
+__device__ __forceinline__ void twiddle16(double2 (&v)[16], double2 w, double2 w2, double2 w3, double2 w4) {
     v[1] = cmul(v[1], w);
     v[2] = cmul(v[2], w2);
     v[3] = cmul(v[3], w3);
@@ -125,21 +130,54 @@ __device__ __forceinline__ void twiddle16(double2 (&v)[16], double2 w) {
     }
 }
 
-// One M-point transform by T = M / 16 threads over z (padded, M + M / 16 words).
-template <int M>
+__device__ __forceinline__ void twiddle16(double2 (&v)[16], double2 w) {
+    const double2 w2 = cmul(w, w), w3 = cmul(w2, w), w4 = cmul(w2, w2);
+    twiddle16(v, w, w2, w3, w4);
+}
+
+__device__ __forceinline__ void twiddle16(double2 (&v)[16], double2 w, double2 w4) {
+    const double2 w2 = cmul(w, w);
+    twiddle16(v, w, w2, cmul(w2, w), w4);
+}
+
+// One M-point transform by T = M / 16 threads over z (padded, M + M / 16 words).  BELT: the fourth
+// powers of the twiddle bases are evaluated, not squared twice, so w^15 carries 6 times a base's
+// rounding instead of 15 times: rms error of the belt's spectra and pixels 3.9 - 5.6e-16 -> 2.2 -
+// 4.5e-16 at Nside 64 - 2048 (single rings 2.3 - 4.6e-16), 1% of the launch.  A cap's convolution
+// (6 - 11e-16, its single ring's direct passes 20 - 220e-16) has no registers to spare for it.
+template <int M, bool BELT = false>
 struct Fft {
     static constexpr int T = M / 16;
     static constexpr int kWords = M + M / 16;
     static constexpr int L2 = M / 16;                    // length after the first pass
     static constexpr int R3 = M > 256 ? M / 256 : 16;     // last length (no twiddles); 256: two passes
     static constexpr bool kMid = M > 256;                 // a middle radix-16 pass over length L2
-    double2 wa, wb;
+    double2 wa, wb;  // twiddle bases
     int t;
 
     __device__ void init(int tid) {
         t = tid;
         wa = cis_pi(2 * t, M, -1.0);
         wb = kMid ? cis_pi(2 * (t % (L2 / 16)), L2, -1.0) : make_double2(1.0, 0.0);
+    }
+    // Twiddles of the first pass and of the middle one.
+    template <bool INV>
+    __device__ __forceinline__ void twiddle_a(double2 (&v)[16]) const {
+        twiddle<INV>(v, wa, t * (2.0 / M));
+    }
+    template <bool INV>
+    __device__ __forceinline__ void twiddle_b(double2 (&v)[16]) const {
+        twiddle<INV>(v, wb, (t % (L2 / 16)) * (2.0 / L2));
+    }
+    template <bool INV>
+    __device__ __forceinline__ static void twiddle(double2 (&v)[16], double2 w, double x) {  // w = e^{-i pi x}
+        if constexpr (INV) w = cconj(w);
+        if constexpr (BELT) {
+            const double2 w4 = cis_minus(4.0 * x);
+            twiddle16(v, w, INV ? cconj(w4) : w4);
+        } else {
+            twiddle16(v, w);
+        }
     }
     // Position of spectrum entry k after the forward passes.
     __device__ static int pos(int k) {
@@ -150,14 +188,14 @@ struct Fft {
     // v: points t + T i, natural order.
     __device__ __forceinline__ void first(double2 (&v)[16], double2* z) const {
         dft<16, false>(v);
-        twiddle16(v, wa);
+        twiddle_a<false>(v);
 #pragma unroll
         for (int j = 0; j < 16; ++j) z[pad(t + T * j)] = v[j];
     }
     __device__ __forceinline__ void last_inv(double2 (&v)[16], const double2* z) const {
 #pragma unroll
         for (int j = 0; j < 16; ++j) v[j] = z[pad(t + T * j)];
-        twiddle16(v, cconj(wa));
+        twiddle_a<true>(v);
         dft<16, true>(v);
     }
     __device__ __forceinline__ int mid_base() const { return (t / (L2 / 16)) * L2 + t % (L2 / 16); }
@@ -167,7 +205,7 @@ struct Fft {
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = z[pad(b + (L2 / 16) * i)];
         dft<16, false>(v);
-        twiddle16(v, wb);
+        twiddle_b<false>(v);
 #pragma unroll
         for (int i = 0; i < 16; ++i) z[pad(b + (L2 / 16) * i)] = v[i];
     }
@@ -176,7 +214,7 @@ struct Fft {
         const int b = mid_base();
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = z[pad(b + (L2 / 16) * i)];
-        twiddle16(v, cconj(wb));
+        twiddle_b<true>(v);
         dft<16, true>(v);
 #pragma unroll
         for (int i = 0; i < 16; ++i) z[pad(b + (L2 / 16) * i)] = v[i];
@@ -502,24 +540,24 @@ __device__ __forceinline__ void cap_ring(const RingArgs& a, int q, bool south, i
 // ------------------------------------------------------------------ belt
 // The middle and last passes of the belt's transform (M = 8192: 16 x 16 x 16 x 2).
 template <int M, bool INV>
-__device__ __forceinline__ void belt_tail(const Fft<M>& F, bool act, double2* z) {
+__device__ __forceinline__ void belt_tail(const Fft<M, true>& F, bool act, double2* z) {
     double2 v[16];
     if constexpr (M <= 4096) {
         if (act) {
             F.tail_load(v, z);
-            Fft<M>::template tail<INV>(v);
+            Fft<M, true>::template tail<INV>(v);
             F.tail_store(v, z);
         }
     } else {
         // (every thread is active) length 32 = 16 x 2: butterfly t takes the words
         // 32 (t / 2) + t % 2 + 2 i, twiddles W32^(t % 2)
         const int base = 32 * (F.t >> 1) + (F.t & 1);
-        const double2 w = cis_pi(F.t & 1, 16, -1.0);
+        const double2 w = cis_pi(F.t & 1, 16, -1.0), w4 = cis_pi(F.t & 1, 4, -1.0);
         if constexpr (!INV) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) v[i] = z[pad(base + 2 * i)];
             dft<16, false>(v);
-            twiddle16(v, w);
+            twiddle16(v, w, w4);
 #pragma unroll
             for (int i = 0; i < 16; ++i) z[pad(base + 2 * i)] = v[i];
             __syncthreads();
@@ -535,7 +573,7 @@ __device__ __forceinline__ void belt_tail(const Fft<M>& F, bool act, double2* z)
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < 16; ++i) v[i] = z[pad(base + 2 * i)];
-            twiddle16(v, cconj(w));
+            twiddle16(v, cconj(w), cconj(w4));
             dft<16, true>(v);
 #pragma unroll
             for (int i = 0; i < 16; ++i) z[pad(base + 2 * i)] = v[i];
@@ -547,7 +585,7 @@ __device__ __forceinline__ void belt_tail(const Fft<M>& F, bool act, double2* z)
 // Belt ring i0 = nside .. 3 nside (spin 2), nside .. 2 nside and its mirror (spin 0).
 template <int M, bool SP2, bool INV>
 __device__ __forceinline__ void belt_ring(const RingArgs& a, int i0, int map, double2* z) {
-    constexpr int T = Fft<M>::T;
+    constexpr int T = Fft<M, true>::T;
     const int tid = threadIdx.x;
     const bool south = SP2 && i0 > 2 * a.nside;
     const RingPair p = ring_pair<SP2>(a.nside, south ? 4 * a.nside - i0 : i0, south);
@@ -556,9 +594,9 @@ __device__ __forceinline__ void belt_ring(const RingArgs& a, int i0, int map, do
     double2* spec = a.spec + (SP2 ? 0 : map * a.smap);
     const bool two = SP2 || p.rs >= 0;
     const bool act = tid < T;
-    Fft<M> F;
+    Fft<M, true> F;
     F.init(act ? tid : 0);
-    auto at = [](int k) { return pad(Fft<M>::pos(k)); };
+    auto at = [](int k) { return pad(Fft<M, true>::pos(k)); };
     double2 v[16];
     if constexpr (!INV) {
         if (act) {
@@ -570,7 +608,7 @@ __device__ __forceinline__ void belt_ring(const RingArgs& a, int i0, int map, do
             F.first(v, z);
         }
         __syncthreads();
-        if constexpr (Fft<M>::kMid) {
+        if constexpr (Fft<M, true>::kMid) {
             if (act) F.mid(z);
             __syncthreads();
         }
@@ -579,7 +617,7 @@ __device__ __forceinline__ void belt_ring(const RingArgs& a, int i0, int map, do
     } else {
         take_rows<SP2>(z, at, 0, p, a.L, spec, a.ld);  // n >= blockDim: no partial words
         belt_tail<M, true>(F, act, z);
-        if constexpr (Fft<M>::kMid) {
+        if constexpr (Fft<M, true>::kMid) {
             if (act) F.mid_inv(z);
             __syncthreads();
         }
