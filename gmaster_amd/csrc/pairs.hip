@@ -349,7 +349,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_ana_pairs(const double2* __restr
         b -= npol;
     }
     const int m = b / nblk, c = b % nblk;
-    const int jhi = min(tab.nact[m], low.pairs(m, jend));
+    if constexpr (SP2) jend = low.pairs(m, jend);
+    const int jhi = min(tab.nact[m], jend);
     const Split sp(jhi - jbeg, T, R);
     const int n = min(sp.spb, sp.total - c * sp.spb);
     if (n <= 0) return;
@@ -556,7 +557,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_syn_pairs(const double2* __restr
         b -= npol;
     }
     const int m = b / nblk, c = b % nblk;
-    jend = low.pairs(m, jend);
+    if constexpr (SP2) jend = low.pairs(m, jend);
     const int jhi = min(tab.nact[m], jend);
     const double2* cf = coef + (table_base(m, tab.L) - m) * K;
     const Split sp(jhi, T, R);
