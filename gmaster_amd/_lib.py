@@ -182,7 +182,8 @@ def query(name, *args):
 
 # Pointers and streams are plain integers (the declared argument types convert them): a transform
 # at Nside 64 passes 78 pointers and asks for the stream 8 times, and with ctypes objects and
-# Stream objects its 18 launches waited for the host (128 us, all of it host time; 122 now, and the GPU works through it without gaps).
+# Stream objects its 18 launches waited for the host (128 us, all of it host time; 122 now, and the
+# GPU works through it without gaps).
 def ptr(t):
     """Device pointer of a tensor (or None -> NULL)."""
     return None if t is None else t.data_ptr()

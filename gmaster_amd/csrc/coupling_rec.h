@@ -12,8 +12,9 @@
 //     f2 = f0 (E^2 - K) / (2 N),   K = 1 + 2 L1 L2,   N^2 = L1 L2 (l1-1)(l1+2)(l2-1)(l2+2),
 // and the l3 recursion Q(l3+1) f2(l3+1) = 4 (2 l3 + 1) f2(l3) - Q(l3) f2(l3-1), solved for the
 // odd degree between two even ones, gives f2(l3+1)^2 = f0(l3)^2 q(l3+1) (E + E')^2 / (16 N^2),
-// E' being E at l3 + 2.  (Both differences of squares are of integers; the recursion of f2 in l3
-// was 29 FP64 operations per two degrees for everything, this is 22.)
+// E' being E at l3 + 2.  (E is an exact integer; E^2 - K is one fused operation, K exact up to l ~ 8192
+// and rounded beyond, which leaves f2 an error of 2^-53 f0.  The recursion of f2 in l3 was 29 FP64
+// operations per two degrees for everything, this is 22.)
 //
 // q(l3) = k (2 l1 + 1 - k) Y with k = l3 - d, Y = (2d + k)(2d + k + 2 l1 + 1): the first factor is
 // the same for every l2 of a row, Y steps by exact integer differences.  The sums sum W'_l3 f^2

@@ -54,10 +54,10 @@ __device__ inline void rescale_lane(F& mu0, F& mu1, int& k) {
 }
 
 // Rescaling of R lanes' recurrences; anyinact (wave-uniform) skips it once every lane is
-// active.  Callers check every 4 degrees, or every 8 where m <= 12288: over 8 degrees from
-// l0 > m a lane grows by at most prod_{k=1..8} (1 + alpha_{m+k}) < 2^55 (alpha_{m+k}^2 <
-// 4 (m + k) / k), so an inactive FP64 lane found just above 2^-300 had stayed below
-// 2^-245: an FP32 zero, and negligible in FP64.
+// active.  Callers check every 4 degrees, or every 8: over 8 degrees from l0 > m a lane grows by
+// at most prod_{k=1..8} (1 + alpha_{m+k}) (alpha_{m+k}^2 < 4 (m + k) / k), 2^55 up to m = 12288,
+// 2^59 up to 24576 and 2^71 up to the largest lmax taken, so an inactive FP64 lane found just
+// above 2^-300 had stayed below 2^-229: an FP32 zero, and negligible in FP64.
 template <int R, typename F>
 __device__ inline void rescale(F (&mu0)[R], F (&mu1)[R], int (&kx)[R], bool& anyinact) {
     if (!anyinact) return;
