@@ -795,9 +795,10 @@ constexpr int kRP = 2;
 // Polar blocks of CHP ring slots beyond the ring pairs below j.
 int polar_blocks(int64_t nside, int64_t j, int CHP) { return (npolar_slots(nside, j) + CHP - 1) / CHP; }
 
-Low low_orders(int64_t nside, int64_t lmax, int64_t jsplit, int CHP) {
+// (of a caller's m < mpol alone: its spin-2 tables need not reach further)
+Low low_orders(int64_t nside, int64_t jsplit, int64_t mpol, int CHP) {
     const int64_t belt = nside + 1, j = belt < jsplit ? belt : jsplit;
-    return Low{(int)(lmax + 1 < kLowOrders ? lmax + 1 : kLowOrders), (int)j, polar_blocks(nside, j, CHP)};
+    return Low{(int)(mpol < kLowOrders ? mpol : kLowOrders), (int)j, polar_blocks(nside, j, CHP)};
 }
 
 }  // namespace
@@ -893,8 +894,7 @@ int check_2(const char* name, int64_t nside, int64_t lmax, int64_t jsplit, int64
     if (nside < 1 || (nside & (nside - 1)) || nside > 8192) return fail(GM_E_ARG, "%s: bad nside", name);
     if (lmax < 2 || lmax > 24 * nside) return fail(GM_E_ARG, "%s: bad lmax %lld", name, (long long)lmax);
     if (jsplit < 1 || jsplit > 2 * nside) return fail(GM_E_ARG, "%s: jsplit outside [1, 2 nside]", name);
-    const int64_t low = lmax + 1 < kLowOrders ? lmax + 1 : kLowOrders;
-    if (mpol < low || mpol > lmax + 1) return fail(GM_E_ARG, "%s: mpol outside [min(%d, lmax + 1), lmax + 1]", name, kLowOrders);
+    if (mpol < 0 || mpol > lmax + 1) return fail(GM_E_ARG, "%s: mpol outside [0, lmax + 1]", name);
     return GM_OK;
 }
 constexpr int kSlots = 4;
@@ -914,7 +914,7 @@ extern "C" int64_t gm_lat2_slots(int64_t nside, int64_t jsplit) {
 extern "C" int64_t gm_lat2_polar_size(int64_t nside, int64_t lmax, int64_t jsplit, int64_t mpol) {
     if (check_2("gm_lat2_polar_size", nside, lmax, jsplit, mpol)) return -1;
     const int CHP = 64 * pair_shape(nside, 2, true, false).NW * kRP;
-    const Low low = low_orders(nside, lmax, jsplit, CHP);
+    const Low low = low_orders(nside, jsplit, mpol, CHP);
     return 4 * (polar_blocks(nside, jsplit, CHP) * table_base(mpol, lmax + 1) + low.nb * table_base(low.n, lmax + 1));
 }
 
@@ -924,7 +924,8 @@ extern "C" int gm_lat2_ana(const double* spec, int64_t ld, int64_t nside, int64_
                            const int32_t* nact2, double* part, double* ppart, int64_t chunk0, void* stream) {
     const char* name = "gm_lat2_ana";
     if (int e = check_2(name, nside, lmax, jsplit, mpol)) return e;
-    if (!spec || !alpha || !smant || !sexp || !nact || !part || !alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2 || !ppart)
+    if (!spec || !alpha || !smant || !sexp || !nact || !part) return fail(GM_E_ARG, "%s: null pointer", name);
+    if (mpol > 0 && (!alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2 || !ppart))
         return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t Lm = lmax + 1;
     if (ld < 2 * Lm - 1) return fail(GM_E_SHAPE, "%s: ld < 2 lmax + 1", name);
@@ -935,7 +936,7 @@ extern "C" int gm_lat2_ana(const double* spec, int64_t ld, int64_t nside, int64_
     const Tables pol{alpha2, gamma2, smant2, sexp2, nact2, (int)Lm};
     const Shape s = pair_shape(nside, 2, true, false);
     const int CH = s.CH, CHP = 64 * s.NW * kRP, nbp = polar_blocks(nside, jsplit, CHP);
-    const Low low = low_orders(nside, lmax, jsplit, CHP);
+    const Low low = low_orders(nside, jsplit, mpol, CHP);
     const int npol = chunk0 == 0 ? low.n * low.nb + ((int)mpol - low.n) * nbp : 0;
     const int jbeg = (int)chunk0 * CH, jend = jbeg + nblk * CH < jsplit ? jbeg + nblk * CH : (int)jsplit;
     return launch_ana<2, true>(name, reinterpret_cast<const double2*>(spec), ld, 0, (int)nside, (int)Lm, tab, jbeg, jend,
@@ -949,7 +950,7 @@ extern "C" int gm_lat2_finish(const double* part, const double* ppart, int64_t n
     const char* name = "gm_lat2_finish";
     if (int e = check_2(name, nside, lmax, jsplit, mpol)) return e;
     if (mode < 0 || mode > 2 || chunk0 < 0) return fail(GM_E_ARG, "%s: bad mode / chunk0", name);
-    if (!part || !nact || !P || !alm_e || !alm_b || !ppart || !nact2 || !P2)
+    if (!part || !nact || !P || !alm_e || !alm_b || (mpol > 0 && (!ppart || !nact2 || !P2)))
         return fail(GM_E_ARG, "%s: null pointer", name);
     const int Lm = (int)lmax + 1;
     const Shape s = pair_shape(nside, 2, true, false);
@@ -957,7 +958,7 @@ extern "C" int gm_lat2_finish(const double* part, const double* ppart, int64_t n
     const int64_t end = (chunk0 + gm_lat2_slots(nside, jsplit)) * s.CH;
     hipLaunchKernelGGL(k_finish_2, dim3((Lm + kFin - 1) / kFin, Lm), dim3(kFin), 0, (hipStream_t)stream, part, ppart, T, s.R,
                        (int)chunk0 * s.CH, (int)(end < jsplit ? end : jsplit), (int)jsplit, nact, P,
-                       polar_blocks(nside, jsplit, CHP), CHP, (int)mpol, low_orders(nside, lmax, jsplit, CHP), nact2, P2, Lm,
+                       polar_blocks(nside, jsplit, CHP), CHP, (int)mpol, low_orders(nside, jsplit, mpol, CHP), nact2, P2, Lm,
                        table_base(mpol, Lm),
                        reinterpret_cast<double2*>(alm_e), reinterpret_cast<double2*>(alm_b), mode);
     return check_launch(name);
@@ -967,7 +968,7 @@ extern "C" int gm_lat2_prep(const double* alm_e, const double* alm_b, const doub
                             int64_t mpol, double* coef, double* pcoef, void* stream) {
     const char* name = "gm_lat2_prep";
     if (int e = check_2(name, 8192, lmax, 1, mpol)) return e;
-    if (!alm_e || !alm_b || !P || !coef || !P2 || !pcoef) return fail(GM_E_ARG, "%s: null pointer", name);
+    if (!alm_e || !alm_b || !P || !coef || (mpol > 0 && (!P2 || !pcoef))) return fail(GM_E_ARG, "%s: null pointer", name);
     const int Lm = (int)lmax + 1;
     hipLaunchKernelGGL(k_prep_2, dim3((Lm + 2 + GM_TABLE_PAD + kFin - 1) / kFin, Lm), dim3(kFin), 0, (hipStream_t)stream,
                        reinterpret_cast<const double2*>(alm_e), reinterpret_cast<const double2*>(alm_b), P, P2, Lm,
@@ -981,7 +982,8 @@ extern "C" int gm_lat2_syn(const double* coef, const double* pcoef, int64_t nsid
                            const int32_t* sexp2, const int32_t* nact2, double* spec, int64_t ld, void* stream) {
     const char* name = "gm_lat2_syn";
     if (int e = check_2(name, nside, lmax, jsplit, mpol)) return e;
-    if (!coef || !alpha || !smant || !sexp || !nact || !spec || !pcoef || !alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2)
+    if (!coef || !alpha || !smant || !sexp || !nact || !spec) return fail(GM_E_ARG, "%s: null pointer", name);
+    if (mpol > 0 && (!pcoef || !alpha2 || !gamma2 || !smant2 || !sexp2 || !nact2))
         return fail(GM_E_ARG, "%s: null pointer", name);
     const int64_t Lm = lmax + 1;
     if (ld < 2 * Lm - 1) return fail(GM_E_SHAPE, "%s: ld < 2 lmax + 1", name);
@@ -990,7 +992,7 @@ extern "C" int gm_lat2_syn(const double* coef, const double* pcoef, int64_t nsid
     const Shape s = pair_shape(nside, 2, true, true);
     const int CH = s.CH, chp = 64 * s.NW * kRP;
     const int nblk = (int)((jsplit + CH - 1) / CH), nbp = polar_blocks(nside, jsplit, chp);
-    const Low low = low_orders(nside, lmax, jsplit, chp);
+    const Low low = low_orders(nside, jsplit, mpol, chp);
     const int npol = low.n * low.nb + ((int)mpol - low.n) * nbp;
     return launch_syn<2, true>(name, reinterpret_cast<const double2*>(coef), (int)nside, (int)Lm, tab, (int)jsplit, nblk,
                                reinterpret_cast<const double2*>(pcoef), pol, nbp, npol, (int)((Lm - mpol) * nbp), low,

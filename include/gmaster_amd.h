@@ -162,10 +162,11 @@ int gm_lat_syn_s(const double* coef, int64_t nside, int64_t lmax, int64_t spin, 
                  const int32_t* nactive, double* spec, int64_t ld, void* stream);
 
 /* ---------------------------------------------------------------- spin 2 on spin-0 rows, FP64
- * The spin-2 transforms of ring pairs j < jsplit (j <= nside, the belt, in the orders m < 8)
- * through the spin-0 rows with weights 1/sin^2 (tables of lmax + 2, nactive in ring pairs), the
- * rings beyond through the spin-2 recurrence (tables of lmax, nactive2 in ring slots; orders
- * m < mpol, the others do not reach them; mpol >= min(8, lmax + 1)).  No counterpart in the
+ * The spin-2 transforms of ring pairs j < jsplit (j <= nside, the belt, in the orders
+ * m < min(8, mpol)) through the spin-0 rows with weights 1/sin^2 (tables of lmax + 2, nactive in
+ * ring pairs), the rings beyond through the spin-2 recurrence (tables of lmax, nactive2 in ring
+ * slots; orders m < mpol, the others do not reach them; 8 or more keeps the error of the lowest
+ * orders that of the spin-2 recurrence).  No counterpart in the
  * reference, which runs a spin-2 recurrence on every ring (gmaster/_native/cuda/march_v2.cu:553-556).
  *   part   gm_lat2_slots x gm_table_size(lmax + 2) x 4 double
  *   ppart  gm_lat2_polar_size double

@@ -123,3 +123,33 @@ def test_low_orders_keep_the_error_of_the_spin2_recurrence(nside, lmax):
             bounds.append(_ratio(got, base, ref))
     print("  analysis: orders 0-7 all %.2f low %.2f, 8-11 all %.2f low %.2f" % tuple(bounds[2:]), flush=True)
     assert max(bounds) < 1.5, bounds
+
+
+@pytest.mark.parametrize("mpol", [0, 3])
+def test_fewer_polar_orders_than_low_ones(mpol):
+    """mpol below the low orders is a caller's choice: every ring pair of the other orders takes the
+    spin-0 rows.  At Nside 8 the weights reach 96 at the first ring, so 96 times the 2e-11 of rows
+    split at sin^2 = 1/64."""
+    import dataclasses
+
+    from gmaster_amd import _lib, sht
+
+    nside, lmax = 8, 20
+    print(f"mpol {mpol}", flush=True)
+    dev = torch.device("cuda", torch.cuda.current_device())
+    L, nring, js = lmax + 1, 4 * nside - 1, 2 * nside
+    p, q = sht.plan2(nside, lmax, dev, False), sht.plan(nside, lmax, 2, dev, False)
+    p = dataclasses.replace(p, jsplit=js, mpol=mpol, nslots=int(_lib.query("gm_lat2_slots", nside, js)),
+                            nchunks=int(_lib.query("gm_lat2_chunks", nside, js)), pol=q,
+                            polar_size=int(_lib.query("gm_lat2_polar_size", nside, lmax, js, mpol)),
+                            ptsize=mpol * (L + 8) - mpol * (mpol - 1) // 2)
+    g = torch.Generator("cuda").manual_seed(mpol)
+    spec = torch.randn((nring, 2 * L - 1), dtype=torch.complex128, device=dev, generator=g)
+    a, b = (torch.empty((2, L * (L + 1) // 2), dtype=torch.complex128, device=dev) for _ in range(2))
+    sht._analysis_2(p, spec, a[0], a[1], 0)
+    sht._analysis_s(q, spec, b[0], b[1], 0)
+    assert float((a - b).abs().max() / b.abs().max()) < 96 * 2e-11
+    s, t = torch.empty_like(spec), torch.empty_like(spec)
+    sht._synthesis_2(p, b[0], b[1], s)
+    sht._synthesis_s(q, b[0], b[1], t)
+    assert float((s - t).abs().max() / t.abs().max()) < 96 * 2e-11
